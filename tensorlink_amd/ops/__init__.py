@@ -216,11 +216,14 @@ def attention_prefill(q, k, v, causal: bool = True,
     scale = scale if scale is not None else 1.0 / math.sqrt(q.shape[-1])
     if not _on_gpu(q):
         return ref.attention_prefill(q, k, v, causal, scale, q_off)
+    grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad
+                                        or v.requires_grad)
     if (q.shape[1] >= 4096 and q_off == 0 and causal
-            and q.shape[1] == k.shape[1]):
-        # long-context full prefill: ROCm flash SDPA measured faster
-        # than the hand-written kernel at S >= 4k (376 vs 259 TF,
-        # profiles/); chunked/q_off windows stay on the HIP kernel
+            and q.shape[1] == k.shape[1]
+            and (grad or q.dtype != torch.bfloat16
+                 or q.shape[-1] not in (64, 128))):
+        # long full prompts that the kernel has no variant for (it is 2.9x
+        # faster where it has one: 7001 rows 440 against 1284 us)
         out = torch.nn.functional.scaled_dot_product_attention(
             q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2),
             is_causal=True, scale=scale, enable_gqa=True)

@@ -27,9 +27,13 @@ void tl_adamw(void* param, const void* grad, void* m, void* v, int64_t n,
 void tl_decode_attn(const void* q, const void* k_cache, const void* v_cache,
                     const void* seq_lens, void* out, int B, int Hq, int Hkv,
                     int Smax, int D, float scale, hipStream_t stream);
-void tl_prefill_attn(const void* q, const void* k, const void* v, void* out,
-                     int B, int Sq, int Skv, int q_off, int Hq, int Hkv,
-                     int D, float scale, int causal, hipStream_t stream);
+int tl_prefill_segments(int Sq, int Skv);
+void tl_prefill_attn(const void* q, const void* k, const void* v,
+                     const void* table, void* out, void* lse, void* po,
+                     void* pml, int64_t kbs, int64_t khs, int kts, int B,
+                     int Sq, int Skv, int q_off, int Hq, int Hkv, int D,
+                     float scale, int causal, int bt_stride,
+                     hipStream_t stream);
 void tl_rope_append(const void* qkv, void* q_out, void* k_cache,
                     void* v_cache, const void* positions,
                     const void* inv_freq, const void* block_table,
@@ -57,10 +61,6 @@ void tl_bump_counter(void* ctr, hipStream_t stream);
 void tl_moe_gemm(const void* x, const void* tok_idx, const void* seg_off,
                  const void* w_ptrs, const void* s_ptrs, void* out, int E,
                  int N, int K, int fp8, hipStream_t stream);
-void tl_prefill_attn_lse(const void* q, const void* k, const void* v,
-                         void* out, void* lse, int B, int Sq, int Skv,
-                         int q_off, int Hq, int Hkv, int D, float scale,
-                         int causal, hipStream_t stream);
 void tl_attn_bwd(const void* q, const void* k, const void* v,
                  const void* dout, const void* lse, const void* delta,
                  void* dq, void* dk, void* dv, int B, int S, int Hq,
@@ -242,21 +242,45 @@ Tensor decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor seq_lens,
   return out;
 }
 
+// k, v: a tensor of rows of D at the given (batch, head, token) strides, or
+// page pools with a table. Split keys go through fp32 partials.
+Tensor prefill_run(const Tensor& q, const Tensor& k, const Tensor& v,
+                   const int* table, int bt_stride, int64_t kbs, int64_t khs,
+                   int64_t kts, int64_t Skv, int64_t Hkv, double scale,
+                   bool causal, int64_t q_off, float* lse) {
+  const int64_t B = q.size(0), Sq = q.size(1), Hq = q.size(2), D = q.size(3);
+  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
+  TORCH_CHECK(Hkv > 0 && Hq % Hkv == 0, "GQA requires Hq % Hkv == 0");
+  TORCH_CHECK(kts <= INT_MAX / 64, "token stride too large");
+  auto out = torch::empty_like(q);
+  if (Skv == 0) {                            // no keys: zeros
+    out.zero_();
+    return out;
+  }
+  const int nseg = lse ? 1 : tl_prefill_segments((int)Sq, (int)Skv);
+  Tensor po, pml;
+  if (nseg > 1) {
+    const auto f32 = q.options().dtype(torch::kFloat);
+    po = torch::empty({nseg * B * Sq * Hq * D}, f32);
+    pml = torch::empty({nseg * B * Sq * Hq * 2}, f32);
+  }
+  tl_prefill_attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), table,
+                  out.data_ptr(), lse, nseg > 1 ? po.data_ptr() : nullptr,
+                  nseg > 1 ? pml.data_ptr() : nullptr, kbs, khs, (int)kts,
+                  (int)B, (int)Sq, (int)Skv, (int)q_off, (int)Hq, (int)Hkv,
+                  (int)D, (float)scale, causal ? 1 : 0, bt_stride, cur_stream());
+  return out;
+}
+
 Tensor prefill_attn(Tensor q, Tensor k, Tensor v, double scale, bool causal,
                     int64_t q_off) {
   CHECK_IN(q, torch::kBFloat16);
   CHECK_IN(k, torch::kBFloat16);
   CHECK_IN(v, torch::kBFloat16);
-  const int B = q.size(0), Sq = q.size(1), Hq = q.size(2), D = q.size(3);
-  const int Skv = k.size(1);
-  const int Hkv = k.size(2);
-  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
-  TORCH_CHECK(q_off + Sq <= Skv || !causal, "q_off + Sq must fit Skv");
-  auto out = torch::empty_like(q);
-  tl_prefill_attn(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                  B, Sq, Skv, (int)q_off, Hq, Hkv, D, (float)scale,
-                  causal ? 1 : 0, cur_stream());
-  return out;
+  const int64_t Skv = k.size(1), Hkv = k.size(2), D = q.size(3);
+  TORCH_CHECK(q_off + q.size(1) <= Skv || !causal, "q_off + Sq must fit Skv");
+  return prefill_run(q, k, v, nullptr, 0, Skv * Hkv * D, D, Hkv * D, Skv, Hkv,
+                     scale, causal, q_off, nullptr);
 }
 
 std::vector<Tensor> prefill_attn_lse(Tensor q, Tensor k, Tensor v,
@@ -264,15 +288,11 @@ std::vector<Tensor> prefill_attn_lse(Tensor q, Tensor k, Tensor v,
   CHECK_IN(q, torch::kBFloat16);
   CHECK_IN(k, torch::kBFloat16);
   CHECK_IN(v, torch::kBFloat16);
-  const int B = q.size(0), Sq = q.size(1), Hq = q.size(2), D = q.size(3);
-  const int Skv = k.size(1);
-  const int Hkv = k.size(2);
-  TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
-  auto out = torch::empty_like(q);
-  auto lse = torch::empty({B, Hq, Sq}, q.options().dtype(torch::kFloat));
-  tl_prefill_attn_lse(q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                      out.data_ptr(), lse.data_ptr(), B, Sq, Skv, 0, Hq,
-                      Hkv, D, (float)scale, causal ? 1 : 0, cur_stream());
+  const int64_t Skv = k.size(1), Hkv = k.size(2), D = q.size(3);
+  auto lse = torch::empty({q.size(0), q.size(2), q.size(1)},
+                          q.options().dtype(torch::kFloat));
+  auto out = prefill_run(q, k, v, nullptr, 0, Skv * Hkv * D, D, Hkv * D, Skv,
+                         Hkv, scale, causal, 0, (float*)lse.data_ptr());
   return {out, lse};
 }
 

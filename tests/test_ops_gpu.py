@@ -165,6 +165,54 @@ def test_prefill_attn_q_off(B, Sq, Skv, q_off, Hq, Hkv, D):
     torch.testing.assert_close(out.float(), out_ref, atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("S,Skv,D", [
+    (1, 1, 128), (31, 31, 64), (33, 97, 128),       # a wave's 32 rows
+    (63, 64, 64), (65, 65, 128), (127, 129, 64),    # a tile's 64 keys
+    (129, 1023, 128), (7, 1024, 64), (130, 1025, 128),   # slices of 1024
+    (512, 2100, 64), (513, 2100, 128),              # cut and not cut
+])
+@pytest.mark.parametrize("scale", [0.09, -0.09])
+def test_prefill_attn_tile_edges(S, Skv, D, scale):
+    """Against fp64; P and the inputs are rounded to bf16 (2^-9 relative),
+    so the 2-norm error of an average of values stays under 4e-3."""
+    ops = _ext()
+    torch.manual_seed(S * 7 + Skv)
+    B, Hq, Hkv = 2, 6, 2
+    q = torch.randn(B, S, Hq, D, device=DEV, dtype=torch.bfloat16)
+    k = torch.randn(B, Skv, Hkv, D, device=DEV, dtype=torch.bfloat16)
+    v = torch.randn(B, Skv, Hkv, D, device=DEV, dtype=torch.bfloat16)
+    out = ops.attention_prefill(q, k, v, scale=scale, q_off=Skv - S)
+    kr = k.double().repeat_interleave(Hq // Hkv, 2).transpose(1, 2)
+    vr = v.double().repeat_interleave(Hq // Hkv, 2).transpose(1, 2)
+    z = q.double().transpose(1, 2) @ kr.transpose(2, 3) * scale
+    late = torch.arange(Skv, device=DEV) > \
+        torch.arange(S, device=DEV)[:, None] + Skv - S
+    want = (z.masked_fill(late, -math.inf).softmax(-1) @ vr).transpose(1, 2)
+    err = (out.double() - want).norm() / want.norm()
+    assert err < 4e-3, float(err)
+
+
+@pytest.mark.parametrize("cuts", [[0, 64, 577, 1089, 1300], [0, 512, 1024],
+                                  [0, 1, 2, 34, 300]])
+def test_prefill_attn_rows_do_not_see_their_portion(cuts):
+    """A row has the same bits whatever portion of the prompt it comes in,
+    with large scores so that the running maximum moves."""
+    ops = _ext()
+    torch.manual_seed(9)
+    n, Hq, Hkv, D = cuts[-1], 4, 2, 128
+    q = 4 * torch.randn(1, n, Hq, D, device=DEV, dtype=torch.bfloat16)
+    k = 4 * torch.randn(1, n, Hkv, D, device=DEV, dtype=torch.bfloat16)
+    v = torch.randn(1, n, Hkv, D, device=DEV, dtype=torch.bfloat16)
+    rows = []
+    for a, b in zip(cuts, cuts[1:]):
+        rows.append(ops.attention_prefill(
+            q[:, a:b], k[:, :b], v[:, :b], q_off=a))
+    whole = [ops.attention_prefill(q[:, a:a + 512], k[:, :a + 512],
+                                   v[:, :a + 512], q_off=a)
+             for a in range(0, n, 512)]
+    assert torch.equal(torch.cat(rows, 1), torch.cat(whole, 1))
+
+
 def test_adamw_matches_torch():
     ops = _ext()
     torch.manual_seed(6)
