@@ -235,9 +235,8 @@ def attention_prefill(q, k, v, causal: bool = True,
 
 class _FlashAttnFn(torch.autograd.Function):
     """Hand-written flash attention for training (gfx950): forward =
-    prefill kernel saving the logsumexp; backward = the two MFMA kernels
-    in ops/csrc/flash_bwd.hip (dKV over key tiles, dQ over query tiles)
-    with Delta = rowsum(dO*O) precomputed in fp32."""
+    prefill kernel saving the logsumexp; backward = the MFMA kernels in
+    ops/csrc/flash_bwd.hip (dKV over key tiles, dQ over query tiles)."""
 
     @staticmethod
     def forward(ctx, q, k, v, causal, scale):
@@ -253,11 +252,9 @@ class _FlashAttnFn(torch.autograd.Function):
     def backward(ctx, dout):
         C = _require_ext()
         q, k, v, out, lse = ctx.saved_tensors
-        delta = (dout.float() * out.float()).sum(-1)          # [B,S,Hq]
-        delta = delta.permute(0, 2, 1).contiguous()           # [B,Hq,S]
         dq, dk, dv = C.attn_bwd(q.contiguous(), k.contiguous(),
-                                v.contiguous(), dout.contiguous(), lse,
-                                delta, ctx.scale, ctx.causal)
+                                v.contiguous(), dout.contiguous(), out, lse,
+                                ctx.scale, ctx.causal)
         return dq, dk, dv, None, None
 
 

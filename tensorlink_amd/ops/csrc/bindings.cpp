@@ -61,11 +61,13 @@ void tl_bump_counter(void* ctr, hipStream_t stream);
 void tl_moe_gemm(const void* x, const void* tok_idx, const void* seg_off,
                  const void* w_ptrs, const void* s_ptrs, void* out, int E,
                  int N, int K, int fp8, hipStream_t stream);
+int tl_attn_bwd_rows(int S);
+int tl_attn_bwd_parts(int B, int S, int Hq, int Hkv);
 void tl_attn_bwd(const void* q, const void* k, const void* v,
-                 const void* dout, const void* lse, const void* delta,
-                 void* dq, void* dk, void* dv, int B, int S, int Hq,
-                 int Hkv, int D, float scale, int causal,
-                 hipStream_t stream);
+                 const void* dout, const void* out, const void* lse,
+                 void* l2, void* delta, void* dq, void* dk, void* dv,
+                 void* pk, void* pv, int B, int S, int Hq, int Hkv, int D,
+                 float scale, int causal, int parts, hipStream_t stream);
 }
 
 namespace {
@@ -297,25 +299,37 @@ std::vector<Tensor> prefill_attn_lse(Tensor q, Tensor k, Tensor v,
 }
 
 std::vector<Tensor> attn_bwd(Tensor q, Tensor k, Tensor v, Tensor dout,
-                             Tensor lse, Tensor delta, double scale,
+                             Tensor out, Tensor lse, double scale,
                              bool causal) {
   CHECK_IN(q, torch::kBFloat16);
   CHECK_IN(k, torch::kBFloat16);
   CHECK_IN(v, torch::kBFloat16);
   CHECK_IN(dout, torch::kBFloat16);
+  CHECK_IN(out, torch::kBFloat16);
   CHECK_IN(lse, torch::kFloat);
-  CHECK_IN(delta, torch::kFloat);
   const int B = q.size(0), S = q.size(1), Hq = q.size(2), D = q.size(3);
   const int Hkv = k.size(2);
   TORCH_CHECK(k.size(1) == S, "training attention needs Sq == Skv");
   TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64 or 128");
+  TORCH_CHECK(Hkv > 0 && Hq % Hkv == 0, "GQA requires Hq % Hkv == 0");
+  TORCH_CHECK(v.sizes() == k.sizes() && k.size(0) == B && k.size(3) == D &&
+                  dout.sizes() == q.sizes() && out.sizes() == q.sizes() &&
+                  lse.numel() == (int64_t)B * Hq * S,
+              "attention backward: shape mismatch");
   auto dq = torch::empty_like(q);
   auto dk = torch::empty_like(k);
   auto dv = torch::empty_like(v);
+  const auto f32 = q.options().dtype(torch::kFloat);
+  auto rows = torch::empty({2, (int64_t)B * Hq * tl_attn_bwd_rows(S)}, f32);
+  const int parts = tl_attn_bwd_parts(B, S, Hq, Hkv);
+  Tensor sums;
+  if (parts > 1) sums = torch::empty({2, parts * k.numel()}, f32);
   tl_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), dout.data_ptr(),
-              lse.data_ptr(), delta.data_ptr(), dq.data_ptr(),
-              dk.data_ptr(), dv.data_ptr(), B, S, Hq, Hkv, D, (float)scale,
-              causal ? 1 : 0, cur_stream());
+              out.data_ptr(), lse.data_ptr(), rows[0].data_ptr(),
+              rows[1].data_ptr(), dq.data_ptr(), dk.data_ptr(),
+              dv.data_ptr(), parts > 1 ? sums[0].data_ptr() : nullptr,
+              parts > 1 ? sums[1].data_ptr() : nullptr, B, S, Hq, Hkv, D,
+              (float)scale, causal ? 1 : 0, parts, cur_stream());
   return {dq, dk, dv};
 }
 
@@ -543,5 +557,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
   mod.def("prefill_attn_lse", &prefill_attn_lse,
           "causal GQA prefill attention returning (out, logsumexp)");
   mod.def("attn_bwd", &attn_bwd,
-          "flash-attention backward: (dq, dk, dv) from saved lse/delta");
+          "flash-attention backward: (dq, dk, dv) from the saved out and lse");
 }

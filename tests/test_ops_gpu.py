@@ -654,6 +654,41 @@ def test_flash_attn_backward(B, S, Hq, Hkv, D, causal):
                                rtol=7e-2)
 
 
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,causal", [
+    (1, 30, 2, 1, 128, True), (2, 31, 4, 2, 64, True),
+    (1, 33, 7, 1, 128, True), (1, 63, 4, 4, 64, False),
+    (2, 65, 6, 2, 128, False), (1, 127, 7, 1, 64, True),
+    (1, 129, 28, 4, 128, True), (1, 700, 14, 2, 128, True),
+    (20, 200, 28, 4, 64, True),      # query heads of a kv head in one block
+])
+@pytest.mark.parametrize("scale", [0.11, -0.11])
+def test_flash_attn_backward_tile_edges(B, S, Hq, Hkv, D, causal, scale):
+    """Against fp64; P, dS, the inputs and the results are rounded to bf16
+    (2^-9 relative), so 2-norm errors stay under 6e-3. Rows of one or two
+    keys are off by more, as Delta comes from the bf16 out and dP - Delta
+    cancels to 2^-9 |dO . O| there (2 rows alone: 0.025); among 30 rows they
+    weigh 1 / 30 and less."""
+    ops = _ext()
+    torch.manual_seed(S + Hq)
+    mk = lambda h: torch.randn(B, S, h, D, device=DEV, dtype=torch.bfloat16)
+    x = [mk(Hq), mk(Hkv), mk(Hkv)]
+    dout = mk(Hq)
+    xs = [t.clone().requires_grad_(True) for t in x]
+    ops.attention_train(*xs, causal=causal, scale=scale).backward(dout)
+    ws = [t.double().requires_grad_(True) for t in x]
+    q = ws[0].transpose(1, 2)
+    k, v = (t.repeat_interleave(Hq // Hkv, 2).transpose(1, 2)
+            for t in ws[1:])
+    z = q @ k.transpose(2, 3) * scale
+    if causal:
+        z = z.masked_fill(torch.ones(S, S, dtype=torch.bool,
+                                     device=DEV).triu(1), -math.inf)
+    (z.softmax(-1) @ v).transpose(1, 2).backward(dout.double())
+    for a, b in zip(xs, ws):
+        err = (a.grad.double() - b.grad).norm() / b.grad.norm()
+        assert err < 6e-3, float(err)
+
+
 def test_training_step_uses_flash_bwd():
     """A PipelineTrainer step runs with the flash kernels on the path
     and the loss decreases."""
