@@ -124,6 +124,15 @@ DEVINLINE unsigned tr16_frag_addr(unsigned panel_base_bytes, int lane) {
          (unsigned)(((q * 8 + (a >> 2)) * 16 + 4 * (a & 3)) * 2);
 }
 
+// Barrier after which every wave's global_load_lds copies are in LDS. The
+// wait is a wave's own: __syncthreads() alone does not always make it (a wave
+// that read nothing from LDS since its copies arrives without it), and other
+// waves would then read what has not landed.
+DEVINLINE void sync_lds_copies() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 #define HIP_CHECK(expr)                                                     \
   do {                                                                      \
     hipError_t _e = (expr);                                                 \

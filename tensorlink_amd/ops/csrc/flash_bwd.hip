@@ -232,7 +232,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 ? 1 : 2) void attn_bwd_dkv_kernel
   if (n > 0) copy(0, 0);
   for (int i = 0; i < n; ++i) {
     const int buf = i & 1;
-    __syncthreads();           // this tile has landed; the other is free
+    sync_lds_copies();         // this tile has landed; the other is free
     if (i + 1 < n) copy(i + 1, buf ^ 1);
     const int t0 = (qt0 + i % nt) * BT;
 #pragma unroll
@@ -359,7 +359,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_bwd_dq_kernel(BwdArgs a) {
   copy(0, 0);
   for (int i = 0; i < n; ++i) {
     const int buf = i & 1, t0 = i * BT;
-    __syncthreads();           // this tile has landed; the other is free
+    sync_lds_copies();         // this tile has landed; the other is free
     if (i + 1 < n) copy(i + 1, buf ^ 1);
 #pragma unroll
     for (int ks = 0; ks < BT; ks += 32) {

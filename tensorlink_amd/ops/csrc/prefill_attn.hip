@@ -205,7 +205,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_attn_kernel(
   copy(0, kv_begin);
   int buf = 0;
   for (int kt0 = kv_begin; kt0 < kv_end; kt0 += BN) {
-    __syncthreads();           // this tile has landed; the other is free
+    sync_lds_copies();         // this tile has landed; the other is free
     if (kt0 + BN < kv_end) copy(buf ^ 1, kt0 + BN);
     // whole tile past this wave's last key: nothing to add
     if (!a.causal || kt0 <= a.q_off + w0 + 31) {
