@@ -271,48 +271,29 @@ class MoEMLP(nn.Module):
         return (self._gu_ptrs, self._down_ptrs, self._gu_scales,
                 self._down_scales)
 
-    def _fused_forward(self, flat, rw, idx, fp8):
-        """Grouped expert GEMMs over expert-sorted (token, slot) pairs;
-        deterministic combine: inverse-permutation gather then a fixed
-        slot-order sum (no atomics — batcher greedy equality holds for
-        MoE models too). hipGraph-capture-safe end to end."""
-        C = ops._require_ext()
-        E, k = self.num_experts, self.top_k
-        T, H = flat.shape
-        P = T * k
-        dev = flat.device
-        gu_p, down_p, gu_s, down_s = self._tables(dev, fp8)
-        fi = idx.reshape(-1)
-        order = fi.argsort(stable=True)
-        # counts via scatter_add (torch.bincount device-syncs, which
-        # breaks hipGraph capture of quantized-MoE decode)
-        counts = torch.zeros(E, device=dev, dtype=torch.long)
-        counts.scatter_add_(0, fi, torch.ones_like(fi))
-        seg = torch.zeros(E + 1, device=dev, dtype=torch.int32)
-        seg[1:] = counts.cumsum(0)
-        pair_tok = (order // k).to(torch.int32)
-        Ie = self.experts[0].inter
-        gu = C.moe_gemm(flat.contiguous(), pair_tok, seg, gu_p, gu_s,
-                        2 * Ie, fp8)
-        act = ops.swiglu_fused(gu)
-        y_pairs = C.moe_gemm(act, None, seg, down_p, down_s, H, fp8)
-        y_pairs = y_pairs * rw.reshape(-1)[order].unsqueeze(1)
-        inv = torch.empty_like(order)
-        inv[order] = torch.arange(P, device=dev, dtype=order.dtype)
-        return y_pairs[inv].view(T, k, H).sum(1)
+    def _fused_forward(self, flat, logits, fp8):
+        """Top-k of the router's logits and grouped expert GEMMs over
+        expert-sorted (token, slot) pairs in one call; deterministic
+        combine: a fixed slot-order sum (no float atomics — batcher greedy
+        equality holds for MoE models too). hipGraph-capture-safe end to
+        end."""
+        gu_p, down_p, gu_s, down_s = self._tables(flat.device, fp8)
+        return ops._require_ext().moe_block(
+            flat.contiguous(), logits.contiguous(), self.top_k, gu_p, down_p,
+            gu_s, down_s, self.experts[0].inter, fp8)
 
     def forward(self, x):
         B, S, H = x.shape
         flat = x.reshape(-1, H)
-        weights, idx = ops.moe_topk_router(self.gate(flat), self.top_k)
-        weights = weights.to(x.dtype)
+        logits = self.gate(flat)
         if (flat.is_cuda and flat.dtype == torch.bfloat16
                 and not torch.is_grad_enabled() and ops.extension_loaded()):
             kind = self._fused_kind()
             if kind is not None:
-                out = self._fused_forward(flat, weights, idx,
-                                          kind == "fp8")
+                out = self._fused_forward(flat, logits, kind == "fp8")
                 return out.reshape(B, S, H)
+        weights, idx = ops.moe_topk_router(logits, self.top_k)
+        weights = weights.to(x.dtype)
         out = torch.zeros_like(flat)
         for e in range(self.num_experts):
             mask = (idx == e)

@@ -58,6 +58,37 @@ void tl_sample(const void* logits, const void* temps, const void* top_ps,
                void* counts, const void* seeds, const void* ctr, void* out,
                uint64_t seed_base, int B, int V, hipStream_t stream);
 void tl_bump_counter(void* ctr, hipStream_t stream);
+int tl_prefill_segments(int Sq, int Skv);
+void tl_prefill_attn(const void* q, const void* k, const void* v,
+                     const void* table, void* out, void* lse, void* po,
+                     void* pml, int64_t kbs, int64_t khs, int kts, int B,
+                     int Sq, int Skv, int q_off, int Hq, int Hkv, int D,
+                     float scale, int causal, int bt_stride,
+                     hipStream_t stream);
+void tl_rope_append(const void* qkv, void* q_out, void* k_cache,
+                    void* v_cache, const void* positions,
+                    const void* inv_freq, const void* block_table,
+                    int64_t T, int row_stride, int S, int Hq, int Hkv,
+                    int D, int Smax, int bt_stride, hipStream_t stream);
+void tl_swiglu_fused(const void* gu, void* out, int64_t N, int I,
+                     hipStream_t stream);
+void tl_decode_attn_mfma(const void* q, const void* k_cache,
+                         const void* v_cache, const void* seq_lens,
+                         const void* block_table, void* out,
+                         void* partial, void* partial_ml, int B, int Hq,
+                         int Hkv, int Smax, int D, float scale, int n_split,
+                         int bt_stride, int per_row, hipStream_t stream);
+void tl_skinny_gemm(const void* x, const void* w, const void* bias,
+                    void* out, void* partial, int M, int N, int K,
+                    int n_split, hipStream_t stream);
+void tl_gemm_tiled(const void* x, const void* w, const void* bias, void* out,
+                   void* partial, int M, int N, int K, int n_split,
+                   hipStream_t stream);
+void tl_sample(const void* logits, const void* temps, const void* top_ps,
+               const void* top_ks, const void* pres, const void* freqs,
+               void* counts, const void* seeds, const void* ctr, void* out,
+               uint64_t seed_base, int B, int V, hipStream_t stream);
+void tl_bump_counter(void* ctr, hipStream_t stream);
 void tl_moe_gemm(const void* x, const void* tok_idx, const void* seg_off,
                  const void* w_ptrs, const void* s_ptrs, void* out, int E,
                  int N, int K, int fp8, hipStream_t stream);
@@ -491,37 +522,6 @@ void bump_sample_counter(Tensor ctr) {
   tl_bump_counter(ctr.data_ptr(), cur_stream());
 }
 
-Tensor moe_gemm(Tensor x, c10::optional<Tensor> tok_idx, Tensor seg_off,
-                Tensor w_ptrs, c10::optional<Tensor> s_ptrs, int64_t N,
-                bool fp8) {
-  CHECK_IN(x, torch::kBFloat16);
-  CHECK_IN(seg_off, torch::kInt);
-  CHECK_IN(w_ptrs, torch::kLong);
-  const int K = x.size(-1);
-  TORCH_CHECK(K % 32 == 0 && N % 64 == 0, "unsupported MoE shape");
-  const int E = w_ptrs.size(0);
-  TORCH_CHECK(seg_off.size(0) == E + 1, "seg_off must be [E+1]");
-  const void* ti = nullptr;
-  int64_t P;
-  if (tok_idx.has_value()) {
-    CHECK_IN(tok_idx.value(), torch::kInt);
-    ti = tok_idx->data_ptr();
-    P = tok_idx->size(0);
-  } else {
-    P = x.size(0);
-  }
-  const void* sp = nullptr;
-  if (fp8) {
-    TORCH_CHECK(s_ptrs.has_value(), "fp8 needs scale pointers");
-    CHECK_IN(s_ptrs.value(), torch::kLong);
-    sp = s_ptrs->data_ptr();
-  }
-  auto out = torch::empty({P, N}, x.options());
-  tl_moe_gemm(x.data_ptr(), ti, seg_off.data_ptr(), w_ptrs.data_ptr(), sp,
-              out.data_ptr(), E, (int)N, K, fp8 ? 1 : 0, cur_stream());
-  return out;
-}
-
 }  // namespace
 
 void register_mix_ops(pybind11::module& mod);  // bindings_mix.cpp
@@ -552,8 +552,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
           "fused penalties/temperature/top-k/top-p sampling, one block/row");
   mod.def("bump_sample_counter", &bump_sample_counter,
           "advance the graph-safe sampling RNG counter");
-  mod.def("moe_gemm", &moe_gemm,
-          "grouped expert GEMM over expert-sorted pair rows");
   mod.def("prefill_attn_lse", &prefill_attn_lse,
           "causal GQA prefill attention returning (out, logsumexp)");
   mod.def("attn_bwd", &attn_bwd,

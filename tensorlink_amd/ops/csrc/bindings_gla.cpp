@@ -35,9 +35,12 @@ void tl_moe_sort(const void* idx, int P, int E, int top, void* seg,
 void tl_grouped_any(const void* x, const void* tok_idx, const void* seg,
                     const void* w, void* out, int P, int E, int N, int K,
                     int is_f32, hipStream_t stream);
-void tl_moe_gemm_stacked(const void* x, const void* tok_idx,
-                         const void* seg_off, const void* w, void* out, int E,
-                         int N, int K, hipStream_t stream);
+void tl_moe_gemm(const void* x, const void* tok, const void* seg,
+                 const void* w_ptrs, const void* w, const void* s_ptrs,
+                 void* out, int64_t P, int E, int N, int K, int fp8,
+                 int gated, hipStream_t stream);
+void tl_moe_softmax_top(const void* z, void* wt, void* idx, int64_t T, int E,
+                        int top, hipStream_t stream);
 void tl_moe_tiles(const void* x, const void* tok, const void* seg,
                   const void* w, void* out, int P, int E, int N, int K,
                   hipStream_t stream);
@@ -265,8 +268,9 @@ Tensor moe_gemm_stacked(Tensor x, c10::optional<Tensor> tok, Tensor seg,
                  out.data_ptr(), (int)P, (int)E, (int)N, (int)K,
                  gla_stream());
   else if (mfma)
-    tl_moe_gemm_stacked(x.data_ptr(), ti, seg.data_ptr(), w.data_ptr(),
-                        out.data_ptr(), (int)E, (int)N, (int)K, gla_stream());
+    tl_moe_gemm(x.data_ptr(), ti, seg.data_ptr(), nullptr, w.data_ptr(),
+                nullptr, out.data_ptr(), P, (int)E, (int)N, (int)K, 0, 0,
+                gla_stream());
   else
     tl_grouped_any(x.data_ptr(), ti, seg.data_ptr(), w.data_ptr(),
                    out.data_ptr(), (int)P, (int)E, (int)N, (int)K, is_f32,
@@ -357,6 +361,73 @@ Tensor moe_experts(Tensor h, Tensor wt, Tensor idx, Tensor gate_up,
   return moe_combine(y, s[2], wt, shared, sg, sg_col, ident, n_real);
 }
 
+// One product of the experts behind a pointer table: w_ptrs [E] addresses of
+// bf16 or fp8 (then with fp32 scales per row) weights [N, K]; gated: [2 N, K],
+// gate rows then up rows, and out is silu(gate) * up.
+Tensor moe_gemm(Tensor x, c10::optional<Tensor> tok, Tensor seg,
+                Tensor w_ptrs, c10::optional<Tensor> s_ptrs, int64_t N,
+                bool fp8, bool gated) {
+  TORCH_CHECK(x.is_cuda() && x.is_contiguous() &&
+                  x.scalar_type() == torch::kBFloat16,
+              "x must be a contiguous bf16 tensor on the GPU");
+  GLA_I32(seg);
+  TORCH_CHECK(w_ptrs.is_cuda() && w_ptrs.is_contiguous() &&
+                  w_ptrs.scalar_type() == torch::kLong,
+              "w_ptrs must be int64 on the GPU");
+  const int64_t K = x.size(-1), E = w_ptrs.size(0);
+  TORCH_CHECK(K % 32 == 0 && N % (gated ? 32 : 64) == 0,
+              "unsupported MoE shape");
+  TORCH_CHECK(seg.size(0) == E + 1, "seg_off must be [E+1]");
+  int64_t P = x.size(0);
+  const void* ti = nullptr;
+  if (tok.has_value()) {
+    GLA_I32(tok.value());
+    P = tok->size(0);
+    ti = tok->data_ptr();
+  }
+  const void* sp = nullptr;
+  if (fp8) {
+    TORCH_CHECK(s_ptrs.has_value(), "fp8 needs scale pointers");
+    TORCH_CHECK(s_ptrs->is_cuda() && s_ptrs->is_contiguous() &&
+                    s_ptrs->scalar_type() == torch::kLong &&
+                    s_ptrs->size(0) == E,
+                "s_ptrs must be int64 [E] on the GPU");
+    sp = s_ptrs->data_ptr();
+  }
+  auto out = torch::empty({P, N}, x.options());
+  tl_moe_gemm(x.data_ptr(), ti, seg.data_ptr(), w_ptrs.data_ptr(), nullptr,
+              sp, out.data_ptr(), P, (int)E, (int)N, (int)K, fp8 ? 1 : 0,
+              gated ? 1 : 0, gla_stream());
+  return out;
+}
+
+// A whole routed block behind its router: softmax and top-k of the logits
+// [T, E], sort, gate|up product with the activation, down product, combine.
+Tensor moe_block(Tensor h, Tensor logits, int64_t top, Tensor gu_ptrs,
+                 Tensor down_ptrs, c10::optional<Tensor> gu_scales,
+                 c10::optional<Tensor> down_scales, int64_t ff, bool fp8) {
+  const int64_t T = h.size(0), W = h.size(1), E = gu_ptrs.size(0);
+  TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() &&
+                  logits.scalar_type() == torch::kBFloat16 &&
+                  logits.dim() == 2 && logits.size(0) == T &&
+                  logits.size(1) == E,
+              "logits must be bf16 [T, E]");
+  TORCH_CHECK(top > 0 && top <= E && top <= tl_moe_max_top() &&
+                  E <= tl_moe_max_experts(),
+              "top or expert count out of range");
+  const auto i32 = h.options().dtype(torch::kInt);
+  auto wt = torch::empty({T, top}, h.options().dtype(torch::kFloat));
+  auto idx = torch::empty({T, top}, i32);
+  tl_moe_softmax_top(logits.data_ptr(), wt.data_ptr(), idx.data_ptr(), T,
+                     (int)E, (int)top, gla_stream());
+  auto s = moe_sort(idx, E);
+  Tensor a = moe_gemm(h, s[1], s[0], gu_ptrs, gu_scales, ff, fp8, true);
+  Tensor y = moe_gemm(a, c10::nullopt, s[0], down_ptrs, down_scales, W, fp8,
+                      false);
+  return moe_combine(y, s[2], wt, c10::nullopt, c10::nullopt, 0, c10::nullopt,
+                     c10::nullopt);
+}
+
 }  // namespace
 
 void register_gla_ops(pybind11::module& mod) {
@@ -373,6 +444,13 @@ void register_gla_ops(pybind11::module& mod) {
   mod.def("moe_sort", &moe_sort, "expert-sorted (token, choice) pairs");
   mod.def("moe_gemm_stacked", &moe_gemm_stacked,
           "grouped product with stacked experts, any size, bf16 or fp32");
+  mod.def("moe_gemm", &moe_gemm,
+          "grouped expert GEMM over expert-sorted pair rows", py::arg("x"),
+          py::arg("tok"), py::arg("seg"), py::arg("w_ptrs"),
+          py::arg("s_ptrs"), py::arg("N"), py::arg("fp8"),
+          py::arg("gated") = false);
+  mod.def("moe_block", &moe_block,
+          "a routed gated block behind its router, in one call");
   mod.def("moe_experts", &moe_experts,
           "sort, grouped products, activation and combine in one call");
   mod.def("moe_combine", &moe_combine,

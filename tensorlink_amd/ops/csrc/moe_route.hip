@@ -177,6 +177,33 @@ __global__ __launch_bounds__(BLOCK) void route_scores_kernel(
   }
 }
 
+// one wave per token, bf16 logits: the `top` most probable experts, weighted
+// by their probabilities over their sum. A NaN or +inf among the logits makes
+// all probabilities, and so the weights, NaN.
+__global__ __launch_bounds__(BLOCK) void route_softmax_kernel(
+    const bf16* __restrict__ z, float* __restrict__ wt,
+    int* __restrict__ idx, int64_t T, int E, int top) {
+  const int64_t t = (int64_t)blockIdx.x * NWAVE + threadIdx.x / WAVE_SIZE;
+  if (t >= T) return;
+  const int lane = threadIdx.x & (WAVE_SIZE - 1);
+  const bf16* zr = z + t * E;
+  float m = -INFINITY;
+  for (int e = lane; e < E; e += WAVE_SIZE) m = fmaxf(m, bf2f(zr[e]));
+  m = wave_reduce_max(m);
+  float sum = 0.f;
+  for (int e = lane; e < E; e += WAVE_SIZE) sum += expf(bf2f(zr[e]) - m);
+  const float inv = 1.f / wave_reduce_sum(sum);
+  float mine;
+  int me;
+  pick_top([&](int e) { return bf2f(zr[e]); }, E, top, mine, me);
+  const float p = lane < top ? expf(mine - m) * inv : 0.f;
+  const float tot = wave_reduce_sum(p);
+  if (lane < top) {
+    wt[t * top + lane] = p / tot;
+    idx[t * top + lane] = min(me, E - 1);
+  }
+}
+
 // one wave per token, logits given
 __global__ __launch_bounds__(BLOCK) void route_select_kernel(
     const float* __restrict__ z, float* __restrict__ wt,
@@ -430,6 +457,16 @@ void tl_moe_route(const void* h, const void* w, const void* z, void* wt,
     hipLaunchKernelGGL(route_logits_kernel<bf16>, grid, block, smem, stream,
                        (const bf16*)h, (const float*)w, (float*)wt,
                        (int*)idx, W, E, top);
+}
+
+// z: bf16 logits [T, E]
+void tl_moe_softmax_top(const void* z, void* wt, void* idx, int64_t T, int E,
+                        int top, hipStream_t stream) {
+  if (T <= 0) return;
+  hipLaunchKernelGGL(route_softmax_kernel,
+                     dim3((unsigned)((T + NWAVE - 1) / NWAVE)), dim3(BLOCK), 0,
+                     stream, (const bf16*)z, (float*)wt, (int*)idx, T, E,
+                     top);
 }
 
 // z: first logit of row 0, rows of stride ldz; corr [E] or null

@@ -573,6 +573,73 @@ def test_moe_gemm_grouped_vs_loop(fp8):
 
 
 @torch.no_grad()
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("T", [1, 3, 31, 70, 600, 1300])
+def test_moe_block_against_fp64(fp8, T):
+    """Every kernel of the rule (few pairs, some, many) with k remainders of
+    32, against fp64 of the same weights; the first rows have the same bits
+    in a call of their own. Gate, up and the activation are rounded to bf16
+    (2^-9 each), so the 2-norm error stays under 8e-3."""
+    C = _ext()._require_ext()
+    from tensorlink_amd.models.quant import quantize_fp8_per_channel
+    torch.manual_seed(52)
+    E, top, H, ff = 6, 2, 192, 96
+    gu = [torch.randn(2 * ff, H, device=DEV, dtype=torch.bfloat16) / H ** 0.5
+          for _ in range(E)]
+    dn = [torch.randn(H, ff, device=DEV, dtype=torch.bfloat16) / ff ** 0.5
+          for _ in range(E)]
+    ptr = lambda ts: torch.tensor([t.data_ptr() for t in ts],
+                                  dtype=torch.int64, device=DEV)
+    if fp8:
+        gq, dq = ([quantize_fp8_per_channel(w) for w in ws]
+                  for ws in (gu, dn))
+        args = [ptr([a for a, _ in gq]), ptr([a for a, _ in dq]),
+                ptr([b for _, b in gq]), ptr([b for _, b in dq])]
+        gd, dd = ([a.double() * b.double()[:, None] for a, b in ws]
+                  for ws in (gq, dq))
+    else:
+        args = [ptr(gu), ptr(dn), None, None]
+        gd, dd = [w.double() for w in gu], [w.double() for w in dn]
+    x = torch.randn(T, H, device=DEV, dtype=torch.bfloat16)
+    z = 3 * torch.randn(T, E, device=DEV, dtype=torch.bfloat16)
+    run = lambda n: C.moe_block(x[:n].contiguous(), z[:n].contiguous(), top,
+                                *args, ff, fp8)
+    out = run(T)
+    w, idx = z.double().softmax(-1).sort(dim=-1, descending=True,
+                                          stable=True)
+    w = w[:, :top] / w[:, :top].sum(-1, keepdim=True)
+    want = torch.zeros(T, H, device=DEV, dtype=torch.double)
+    for e in range(E):
+        at, slot = (idx[:, :top] == e).nonzero(as_tuple=True)
+        g, u = (x[at].double() @ gd[e].t()).chunk(2, -1)
+        want.index_add_(0, at, w[at, slot, None] * (
+            (torch.nn.functional.silu(g) * u) @ dd[e].t()))
+    err = (out.double() - want).norm() / want.norm()
+    assert err < 8e-3, float(err)
+    assert torch.equal(run(min(T, 3)), out[:3])
+
+
+@torch.no_grad()
+def test_moe_block_logits_that_are_not_numbers():
+    """A row with a NaN or +inf logit is NaN throughout, as softmax has it;
+    the other rows are untouched."""
+    C = _ext()._require_ext()
+    torch.manual_seed(53)
+    E, H, ff = 4, 64, 32
+    gu, dn = (torch.randn(E, *s, device=DEV, dtype=torch.bfloat16) / 8
+              for s in ((2 * ff, H), (H, ff)))
+    ptr = lambda t: torch.tensor([t[e].data_ptr() for e in range(E)],
+                                 dtype=torch.int64, device=DEV)
+    x = torch.randn(5, H, device=DEV, dtype=torch.bfloat16)
+    z = torch.randn(5, E, device=DEV, dtype=torch.bfloat16)
+    good = C.moe_block(x, z, 2, ptr(gu), ptr(dn), None, None, ff, False)
+    z[1, 2], z[3] = math.inf, math.nan
+    out = C.moe_block(x, z, 2, ptr(gu), ptr(dn), None, None, ff, False)
+    assert out[[1, 3]].isnan().all()
+    assert torch.equal(out[[0, 2, 4]], good[[0, 2, 4]])
+
+
+@torch.no_grad()
 def test_moe_fused_block_matches_loop():
     """MoEMLP's fused grouped path equals the per-expert loop."""
     from tensorlink_amd.models.configs import get_config
