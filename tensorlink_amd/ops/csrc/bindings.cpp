@@ -49,10 +49,10 @@ void tl_decode_attn_mfma(const void* q, const void* k_cache,
                          int bt_stride, int per_row, hipStream_t stream);
 void tl_skinny_gemm(const void* x, const void* w, const void* bias,
                     void* out, void* partial, int M, int N, int K,
-                    int n_split, hipStream_t stream);
+                    int n_split, int k_per, hipStream_t stream);
 void tl_gemm_tiled(const void* x, const void* w, const void* bias, void* out,
                    void* partial, int M, int N, int K, int n_split,
-                   hipStream_t stream);
+                   int k_per, hipStream_t stream);
 void tl_sample(const void* logits, const void* temps, const void* top_ps,
                const void* top_ks, const void* pres, const void* freqs,
                void* counts, const void* seeds, const void* ctr, void* out,
@@ -80,10 +80,10 @@ void tl_decode_attn_mfma(const void* q, const void* k_cache,
                          int bt_stride, int per_row, hipStream_t stream);
 void tl_skinny_gemm(const void* x, const void* w, const void* bias,
                     void* out, void* partial, int M, int N, int K,
-                    int n_split, hipStream_t stream);
+                    int n_split, int k_per, hipStream_t stream);
 void tl_gemm_tiled(const void* x, const void* w, const void* bias, void* out,
                    void* partial, int M, int N, int K, int n_split,
-                   hipStream_t stream);
+                   int k_per, hipStream_t stream);
 void tl_sample(const void* logits, const void* temps, const void* top_ps,
                const void* top_ks, const void* pres, const void* freqs,
                void* counts, const void* seeds, const void* ctr, void* out,
@@ -429,22 +429,17 @@ static int gemm_split_target() {
   return t;
 }
 
-static int gemm_n_split(int N, int K) {
-  if (N >= 65536) {
-    // 256x256-tile class (gemm_tiled_sq, lm_head widths): enough
-    // column panels to fill the chip without splitting
-    int n_split = 1;
-    while (((N + 255) / 256) * n_split < gemm_split_target() &&
-           n_split < 16 && (K / 64) / (n_split * 2) >= 16)
-      n_split <<= 1;
-    return n_split;
-  }
-  // split K so (N/64)*n_split lands near the target block count
-  int n_split = 1;
-  while ((N / 64) * n_split < gemm_split_target() && n_split < 8 &&
-         (K / 32) / (n_split * 2) >= 2)
-    n_split <<= 1;
-  return n_split;
+struct GemmSplit {
+  int n, k_per;
+};
+
+static GemmSplit gemm_split(int N, int K) {
+  const int steps = (K + 255) / 256, panels = N / 64;
+  const int most = gemm_split_target() / panels;
+  const int n = std::min(most >= 4 ? 4 : most >= 2 ? 2 : 1, steps);
+  if (n <= 1) return {1, K};
+  const int per = (steps + n - 1) / n;
+  return {(steps + per - 1) / per, per * 256};
 }
 
 Tensor skinny_gemm(Tensor x, Tensor w, c10::optional<Tensor> bias) {
@@ -463,7 +458,7 @@ Tensor skinny_gemm(Tensor x, Tensor w, c10::optional<Tensor> bias) {
     CHECK_IN(bias.value(), torch::kBFloat16);
     bp = bias->data_ptr();
   }
-  const int n_split = gemm_n_split(N, K);
+  const auto [n_split, k_per] = gemm_split(N, K);
   Tensor partial;
   void* pp = nullptr;
   if (n_split > 1) {
@@ -473,10 +468,10 @@ Tensor skinny_gemm(Tensor x, Tensor w, c10::optional<Tensor> bias) {
   }
   if (M <= 64)
     tl_skinny_gemm(x.data_ptr(), w.data_ptr(), bp, out.data_ptr(), pp,
-                   (int)M, N, K, n_split, cur_stream());
+                   (int)M, N, K, n_split, k_per, cur_stream());
   else
     tl_gemm_tiled(x.data_ptr(), w.data_ptr(), bp, out.data_ptr(), pp,
-                  (int)M, N, K, n_split, cur_stream());
+                  (int)M, N, K, n_split, k_per, cur_stream());
   return out;
 }
 

@@ -1,20 +1,29 @@
-// Skinny-M GEMM for the decode path: out[M,N] = x[M,K] @ W[N,K]^T (+bias).
+// Skinny-M GEMM for the decode path: out[M,N] = x[M,K] @ W[N,K]^T (+bias),
+// M <= 64.
 //
 // torch Linear stores W as [N, K] row-major, so both operands are
-// k-contiguous — the same A·B^T fragment pattern as QK^T. At decode M
-// (<= 256 rows) the GEMM is pure W-streaming.
+// k-contiguous. At decode M the GEMM is pure W-streaming: what bounds it is
+// how many bytes of W are in flight and how few launches surround it.
 //
-// v3 geometry (measured on MI355X):
-//   v1 gridded over M: every W panel re-streamed per M-tile -> 0.4 TB/s.
-//   v2 looped M-tiles with fragment-shaped x loads straight from global:
-//   16 scatter-line loads per W load -> TA transaction-bound, 0.23-0.37
-//   TB/s (the guide's "fragment-shaped x" trap).
-//   v3 stages the x k-slab into LDS ONCE per block with full-line
-//   coalesced loads (+16 B row pad -> conflict-free ds_read_b128
-//   A-fragments), shared by all 4 waves x all M-tiles; W streams straight
-//   from HBM exactly once chip-wide.
-// Grid (N/64, SPLITK); block = 4 waves; wave w owns columns w*16; SPLITK
-// slices K when N/64 can't fill the chip (fp32 partials + reduce kernel).
+// A block covers 64 rows of W and all rows of x. Both go to LDS by
+// global_load_lds (256 contiguous bytes per row, 16-byte slots permuted by
+// row, so the ds_read_b128 meet no conflicts), three steps of 128 k ahead in
+// four buffers. The copies are counted: a step waits for the oldest only, with
+// one barrier. W through registers instead is 64 bytes per row and load, and
+// the compiler then drains all copies at each use. A wave owns 16 rows of W
+// (the A operand, so a lane ends with four neighbouring columns of a row).
+// Grid (N/64, n_split): K is cut in 2 or 4 where N/64 leaves CUs without a
+// block (fp32 partials + reduce kernel), at multiples of 256.
+//
+// Measured on MI355X, 1 / 16 / 64 rows, reduce included (before: W through
+// registers, one step ahead, a barrier that drained it): 3584 x 18944 44 / 45
+// / 53 -> 28 / 28 / 35 us (4.9 TB/s), 4096 x 12288 46 / 47 / 53 -> 21 / 22 /
+// 25, 4608 x 3584 19 / 19 / 22 -> 11 / 11 / 15, 152064 x 3584 241 / 253 / 291
+// -> 179 / 186 / 232 (6.1 TB/s). Cuts inside the block, each with a wave's own
+// buffers and no partials, were slower (44 us on 3584 x 18944).
+//
+// Contract with gemm_tiled.hip: every row sums K in 32-wide
+// mfma_f32_16x16x32_bf16 steps in order within a cut, and the cuts in order.
 
 #include "common.hpp"
 
@@ -24,168 +33,170 @@ constexpr int BLOCK = 256;
 
 using f32x4 = __attribute__((ext_vector_type(4))) float;
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 
-template <int MT, int HAS_BIAS, int SPLIT>
-__global__ __launch_bounds__(BLOCK, 2) void skinny_gemm_kernel(
+template <int N>
+DEVINLINE void waitcnt_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+constexpr int XK = 128;              // k per step
+constexpr int NB = 4;                // buffers
+
+template <int MT, int SPLIT>
+__global__ __launch_bounds__(BLOCK) void skinny_gemm_kernel(
     const bf16* __restrict__ x,     // [M, K]
     const bf16* __restrict__ w,     // [N, K]
     const bf16* __restrict__ bias,  // [N] or null
     bf16* __restrict__ out,         // [M, N]
-    float* __restrict__ partial,    // [SPLITK, M, N] when SPLIT
-    int M, int N, int K, int n_split) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int col = lane & 15;
-  const int quad = lane >> 4;
-  const int oc = blockIdx.x * 64 + wave * 16 + col;   // output column
+    float* __restrict__ partial,    // [n_split, M, N] when SPLIT
+    int M, int N, int K, int k_per) {
+  constexpr int R = MT * 16 + 64;            // rows of a buffer: x, then w
+  constexpr int CPW = R / 16;                // copies of four rows per wave
+  __shared__ bf16 lds[NB][R][XK];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, quad = lane >> 4;
+  const int n0 = blockIdx.x * 64 + wave * 16;
+  const int kb = SPLIT ? blockIdx.y * k_per : 0;
+  const int ke = SPLIT ? min(K, kb + k_per) : K;
 
-  const int m_tiles = (M + 15) / 16;
-  const int split = SPLIT ? blockIdx.y : 0;
-  const int k_per = SPLIT ? (((K + 63) / 64 + n_split - 1) / n_split) * 64 : K;
-  const int k_begin = split * k_per;
-  const int k_end = min(K, k_begin + k_per);
-
-  // Double-buffered x slab staged by global_load_lds (HBM->LDS DMA: no
-  // staging registers — register staging at MT=16 spilled 272 B/lane).
-  // glds writes lane-linear (base + lane*16), so the LDS image is
-  // unpadded; the bank swizzle moves to the SOURCE address (guide rule
-  // 21): physical 16-B slot p of row r holds logical k-slot p^(r&7), and
-  // the fragment read applies the same XOR — 8-way read conflicts drop to
-  // 2-way with FETCH-neutral sources (the XOR permutes within one row's
-  // 128 B).
-  __shared__ bf16 x_lds[2][MT * 16][64];
-
+  const bf16* src[CPW];
+  int off[CPW];
+#pragma unroll
+  for (int g = 0; g < CPW; ++g) {
+    const int r = (wave * CPW + g) * 4 + quad;
+    src[g] = r < MT * 16
+                 ? x + (int64_t)min(r, M - 1) * K
+                 : w + ((int64_t)blockIdx.x * 64 + r - MT * 16) * K;
+    off[g] = (col ^ (r & 15)) * 8;
+  }
+  auto copy = [&](int i) {
+    const int k0 = kb + i * XK;
+#pragma unroll
+    for (int g = 0; g < CPW; ++g)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(
+              src[g] + min(k0 + off[g], K - 8)),
+          (__attribute__((address_space(3))) void*)(
+              &lds[i & (NB - 1)][(wave * CPW + g) * 4][0]),
+          16, 0, 0);
+  };
   f32x4 acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  const bf16* wrow = w + (int64_t)oc * K;   // this lane's W row
-
-  constexpr int GPW = MT > 1 ? MT / 2 : 1;  // glds chunks per wave
-  const int l8 = lane >> 3, c8 = lane & 7;
-
-#define SG_GLDS_TILE(bufi, k0)                                              \
-  if ((k0) < K) {                                                           \
-    _Pragma("unroll") for (int g = 0; g < GPW; ++g) {                       \
-      const int chunk = wave * GPW + g;      /* 8 rows per 1-KB chunk */    \
-      if (chunk >= MT * 2) break; /* MT=1: only 2 chunks (wave-uniform) */  \
-      const int row = chunk * 8 + l8;                                       \
-      const int xr = min(row, M - 1);                                       \
-      const int kc = min((k0) + (c8 ^ (row & 7)) * 8, K - 8);               \
-      auto gsrc = (const __attribute__((address_space(1))) void*)(          \
-          x + (int64_t)xr * K + kc);                                        \
-      auto ldst = (__attribute__((address_space(3))) void*)(                \
-          &x_lds[bufi][chunk * 8][0]);                                      \
-      __builtin_amdgcn_global_load_lds(gsrc, ldst, 16, 0, 0);               \
-    }                                                                       \
+  auto product = [&](int buf, int t) {       // 32 k
+    const int s = ((t * 4 + quad) ^ col) * 8;
+    const bf16x8_t wf = *reinterpret_cast<const bf16x8_t*>(
+        &lds[buf][MT * 16 + wave * 16 + col][s]);
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          wf, *reinterpret_cast<const bf16x8_t*>(&lds[buf][m * 16 + col][s]),
+          acc[m], 0, 0, 0);
+  };
+  const int whole = (ke - kb) / XK;
+  const int ns = (ke - kb + XK - 1) / XK;
+  auto arrive = [&](int i) {                 // step i is in LDS, i - 1 free
+    if (i + 2 < ns)
+      waitcnt_vm<2 * CPW>();
+    else if (i + 1 < ns)
+      waitcnt_vm<CPW>();
+    else
+      waitcnt_vm<0>();
+    __builtin_amdgcn_s_barrier();
+    if (i + 3 < ns) copy(i + 3);
+  };
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (i < ns) copy(i);
+  for (int i = 0; i < whole; ++i) {
+    arrive(i);
+#pragma unroll
+    for (int t = 0; t < XK / 32; ++t) product(i & (NB - 1), t);
+  }
+  if (whole < ns) {                          // less than a step is left
+    arrive(whole);
+    for (int t = 0; t < (ke - kb - whole * XK) / 32; ++t)
+      product(whole & (NB - 1), t);
   }
 
-  SG_GLDS_TILE(0, k_begin);
-  int buf = 0;
-  for (int k0 = k_begin; k0 < k_end; k0 += 64) {
-    __syncthreads();                          // drains this tile's glds
-    if (k0 + 64 < k_end)
-      SG_GLDS_TILE(buf ^ 1, k0 + 64);         // in flight under compute
-    const int tile_k = min(64, k_end - k0);
+  // lane: columns n0 + quad * 4 + 0..3 of row m * 16 + col
+  const int n = n0 + quad * 4;
+  f32x4 b = (f32x4){0.f, 0.f, 0.f, 0.f};
+  if (!SPLIT && bias) {
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      if (kk * 32 < tile_k) {
-        bf16x8_t bfrag = *reinterpret_cast<const bf16x8_t*>(
-            wrow + k0 + kk * 32 + quad * 8);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          // unconditional across MT (dispatch picks smallest MT >=
-          // m_tiles; guarded acc updates made the compiler home the
-          // accumulator array in scratch)
-          const int row = m * 16 + col;
-          const int slot = (kk * 4 + quad) ^ (row & 7);
-          bf16x8_t afrag = *reinterpret_cast<const bf16x8_t*>(
-              &x_lds[buf][row][slot * 8]);
-          acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              afrag, bfrag, acc[m], 0, 0, 0);
-        }
-      }
-    }
-    buf ^= 1;
+    for (int r = 0; r < 4; ++r) b[r] = bf2f(bias[n + r]);
   }
-#undef SG_GLDS_TILE
-
-  // epilogue: lane holds C[row=quad*4+r][col] per m-tile
-  const float b = HAS_BIAS ? bf2f(bias[oc]) : 0.f;
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
+    const int row = m * 16 + col;
+    if (row >= M) continue;
+    if (SPLIT) {
+      *reinterpret_cast<f32x4*>(
+          partial + ((int64_t)blockIdx.y * M + row) * N + n) = acc[m];
+    } else {
+      bf16x4_t o;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int orow = m * 16 + quad * 4 + r;
-      if (orow < M) {
-        if (SPLIT)
-          partial[((int64_t)split * M + orow) * N + oc] = acc[m][r];
-        else
-          out[(int64_t)orow * N + oc] = f2bf(acc[m][r] + b);
-      }
+      for (int r = 0; r < 4; ++r) o[r] = (__bf16)(acc[m][r] + b[r]);
+      *reinterpret_cast<bf16x4_t*>(out + (int64_t)row * N + n) = o;
     }
   }
 }
 
-template <int HAS_BIAS>
-__global__ void skinny_reduce_kernel(const float* __restrict__ partial,
-                                     const bf16* __restrict__ bias,
-                                     bf16* __restrict__ out, int64_t MN,
-                                     int N, int n_split) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// N is a multiple of 64: four columns per thread
+__global__ __launch_bounds__(BLOCK) void skinny_reduce_kernel(
+    const float* __restrict__ partial, const bf16* __restrict__ bias,
+    bf16* __restrict__ out, int64_t MN, int N, int n_split) {
+  const int64_t i = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) * 4;
   if (i >= MN) return;
-  float acc = 0.f;
-  for (int s = 0; s < n_split; ++s) acc += partial[s * MN + i];
-  if (HAS_BIAS) acc += bf2f(bias[i % N]);
-  out[i] = f2bf(acc);
+  f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < n_split; ++s)
+    acc += *reinterpret_cast<const f32x4*>(partial + s * MN + i);
+  bf16x4_t o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float b = bias ? bf2f(bias[i % N + r]) : 0.f;
+    o[r] = (__bf16)(bias ? acc[r] + b : acc[r]);
+  }
+  *reinterpret_cast<bf16x4_t*>(out + i) = o;
 }
 
 }  // namespace
 
 extern "C" {
 
-// partial: scratch [n_split * M * N] floats (only read when n_split > 1).
+// out = the sum over the cuts, in order, plus bias
+void tl_gemm_reduce(const void* partial, const void* bias, void* out,
+                    int64_t MN, int N, int n_split, hipStream_t stream) {
+  hipLaunchKernelGGL(skinny_reduce_kernel,
+                     dim3((uint32_t)((MN / 4 + BLOCK - 1) / BLOCK)),
+                     dim3(BLOCK), 0, stream, (const float*)partial,
+                     (const bf16*)bias, (bf16*)out, MN, N, n_split);
+}
+
+// partial: scratch [n_split * M * N] floats (only used when n_split > 1)
 void tl_skinny_gemm(const void* x, const void* w, const void* bias,
                     void* out, void* partial, int M, int N, int K,
-                    int n_split, hipStream_t stream) {
-  const int m_tiles = (M + 15) / 16;
-  const int split = n_split > 1 ? 1 : 0;
-  dim3 grid(N / 64, n_split), block(BLOCK);
-#define DISPATCH(MT)                                                        \
-  do {                                                                      \
-    if (split) {                                                            \
-      hipLaunchKernelGGL((skinny_gemm_kernel<MT, 0, 1>), grid, block, 0,    \
-                         stream, (const bf16*)x, (const bf16*)w, nullptr,   \
-                         (bf16*)out, (float*)partial, M, N, K, n_split);    \
-    } else if (bias) {                                                      \
-      hipLaunchKernelGGL((skinny_gemm_kernel<MT, 1, 0>), grid, block, 0,    \
-                         stream, (const bf16*)x, (const bf16*)w,            \
-                         (const bf16*)bias, (bf16*)out, nullptr, M, N, K,   \
-                         1);                                                \
-    } else {                                                                \
-      hipLaunchKernelGGL((skinny_gemm_kernel<MT, 0, 0>), grid, block, 0,    \
-                         stream, (const bf16*)x, (const bf16*)w, nullptr,   \
-                         (bf16*)out, nullptr, M, N, K, 1);                  \
-    }                                                                       \
+                    int n_split, int k_per, hipStream_t stream) {
+  const dim3 grid(N / 64, n_split), block(BLOCK);
+#define TL_SG(MT)                                                            \
+  do {                                                                       \
+    if (n_split > 1)                                                         \
+      hipLaunchKernelGGL((skinny_gemm_kernel<MT, 1>), grid, block, 0,        \
+                         stream, (const bf16*)x, (const bf16*)w, nullptr,    \
+                         nullptr, (float*)partial, M, N, K, k_per);          \
+    else                                                                     \
+      hipLaunchKernelGGL((skinny_gemm_kernel<MT, 0>), grid, block, 0,        \
+                         stream, (const bf16*)x, (const bf16*)w,             \
+                         (const bf16*)bias, (bf16*)out, nullptr, M, N, K,    \
+                         K);                                                 \
   } while (0)
-  if (m_tiles <= 1) DISPATCH(1);
-  else if (m_tiles <= 2) DISPATCH(2);
-  else if (m_tiles <= 4) DISPATCH(4);
-  else if (m_tiles <= 8) DISPATCH(8);
-  else DISPATCH(16);
-#undef DISPATCH
-  if (split) {
-    const int64_t MN = (int64_t)M * N;
-    dim3 rgrid((uint32_t)((MN + 255) / 256)), rblock(256);
-    if (bias)
-      hipLaunchKernelGGL((skinny_reduce_kernel<1>), rgrid, rblock, 0, stream,
-                         (const float*)partial, (const bf16*)bias,
-                         (bf16*)out, MN, N, n_split);
-    else
-      hipLaunchKernelGGL((skinny_reduce_kernel<0>), rgrid, rblock, 0, stream,
-                         (const float*)partial, nullptr, (bf16*)out, MN, N,
-                         n_split);
-  }
+  if (M <= 16) TL_SG(1);
+  else if (M <= 32) TL_SG(2);
+  else TL_SG(4);
+#undef TL_SG
+  if (n_split > 1)
+    tl_gemm_reduce(partial, bias, out, (int64_t)M * N, N, n_split, stream);
 }
 
 }  // extern "C"
