@@ -359,6 +359,27 @@ def test_tl_gemm(M, N, K, bias):
     torch.testing.assert_close(out.float(), ref, atol=5e-2, rtol=5e-2)
 
 
+@pytest.mark.parametrize("N,K", [
+    (64, 32), (128, 160), (320, 544), (64, 2080),      # k remainders, 4 cuts
+    (8192, 800), (16384, 288), (65600, 96),            # 2 cuts, none, wide
+])
+@pytest.mark.parametrize("bias", [False, True])
+def test_tl_gemm_edges(N, K, bias):
+    """Every kernel of the family at the edges of its rows against fp64, and
+    the same bits from all of them. The result is rounded to bf16 (2^-9) and
+    summed in fp32: the 2-norm error stays under 3e-3."""
+    C = _ext()._require_ext()
+    torch.manual_seed(N + K)
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) / K ** 0.5
+    b = torch.randn(N, device=DEV, dtype=torch.bfloat16) if bias else None
+    x = torch.randn(300, K, device=DEV, dtype=torch.bfloat16)
+    full = C.skinny_gemm(x, w, b)
+    want = x.double() @ w.double().t() + (b.double() if bias else 0)
+    assert (full.double() - want).norm() / want.norm() < 3e-3
+    for M in (1, 16, 17, 32, 33, 64, 65, 128, 129, 257):
+        assert torch.equal(C.skinny_gemm(x[:M].contiguous(), w, b), full[:M])
+
+
 def test_decode_attn_batch_independence():
     """A row's decode attention is bitwise identical whatever batch it is
     in (per-row flash-decode split from its own length — common.hpp
