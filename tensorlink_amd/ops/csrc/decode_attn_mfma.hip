@@ -1,261 +1,328 @@
-// MFMA decode attention (v2) for gfx950.
+// MFMA decode attention for gfx950.
 //
-// The v1 kernel (decode_attn.hip) is VALU-bound: ~85 VALU ops per 64 B of
-// KV streamed caps it at ~2.6 TB/s effective (profiles/). Here the score
-// and PV math run on the matrix cores instead:
+// One block serves all G <= 16 query heads of one kv head over one slice of a
+// sequence, so K and V are read once. What bounds it is how many bytes of K
+// and V are in flight: every wave copies tiles of 32 keys to LDS buffers of
+// its own with global_load_lds, one tile ahead, waits for its own copies only
+// and meets the others once, at the end.
 //
-//   grid (B, Hkv, SPLIT): ONE block covers ALL G <= 16 query heads of one
-//   kv head (single pass over the K/V slab — v1 needed ceil(G/4) passes),
-//   with the MFMA M-dimension = query heads.
-//   Per 16-key tile: QK^T = mfma_f32_16x16x32_bf16 over D/32 k-chunks,
-//   where the B-fragment IS the natural K layout (lane l reads 16 B of key
-//   l&15 at d-offset (l>>4)*8 — no LDS staging for K). V is staged
-//   transposed through LDS (pad stride 40 elems: 16-B aligned, 20-dword
-//   row stride is conflict-free over 16 rows) so the PV B-fragment is a
-//   contiguous ds_read_b128. P round-trips through a small LDS tile to
-//   convert C-layout -> A-layout.
+// The scores are formed transposed, S^T = K Q^T (16x16x32 MFMA, a lane holds 8
+// keys of ONE head), so the row maximum is in-lane plus two exchanges, and the
+// accumulators of two 16-key tiles ARE the B operand of O^T = V^T P^T once its
+// 32 keys are counted as 4q..4q+3, 16+4q..16+4q+3 for quad q; V^T comes in
+// that order from ds_read_b64_tr_b16. P does not pass through LDS.
 //
-// Flash-decode SPLIT: for small B*Hkv the seq dim is partitioned across
-// SPLIT blocks writing (m, l, o) partials; a tiny combine kernel merges.
+// Flash-decode SPLIT: a long row is cut into slices (tl_split_for_len) in
+// blocks that write (m, l, o) partials; a combine kernel merges them in order.
+//
+// Measured on MI355X, D 128 (before: 16-key tiles, K loaded where it is used,
+// V through LDS stores, no copy in flight over a tile): 1 sequence of 513 keys,
+// 4 kv heads, 16.5 -> 8.6 us; 8 of 1000, 8 kv heads, 32 -> 14; 48 of 1958 96
+// -> 74 (5.2 TB/s); 256 of 577, 4 kv heads, 66 -> 62 (4.9 TB/s); 2 of 32400 84
+// -> 63.
 
 #include "common.hpp"
 
 namespace {
 
-constexpr int BLOCK = 256;
 constexpr int NWAVE = 4;
-constexpr int KT = 16;            // keys per MFMA tile
+constexpr int KT = 32;            // keys per tile
 
 using f32x4 = __attribute__((ext_vector_type(4))) float;
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
-// out layout when SPLIT > 1: partial [B, Hq, SPLIT, D] float, ml [B, Hq,
-// SPLIT, 2] float (m, l). SPLIT == 1 writes bf16 out directly.
-// PAGED: k_cache/v_cache are page pools [n_pages, Hkv, PAGE, D] and
-// block_table [B, bt_stride] maps position/PAGE -> page id (PAGE = 128).
+constexpr float LOG2E = 1.4426950408889634f;
+
+// 16-byte slot permutations within a row of D elements: K is read 16 rows at
+// one slot, V four rows at 32 bytes (the quads' row groups alternate halves).
+template <int D>
+DEVINLINE int k_perm(int row) {
+  return D == 128 ? (row & 15) : ((row >> 1) & 7);
+}
+template <int D>
+DEVINLINE int v_perm(int row) {
+  return D == 128 ? (((row & 3) << 1) | (((row >> 2) & 1) << 3))
+                  : ((((row >> 1) & 1) << 1) | (((row >> 2) & 1) << 2));
+}
+
+// Transposed reads of 32 keys x 4 tiles of 16 columns; the wait is inside, as
+// a read in flight must not have its registers reused.
+struct VFrag {
+  uint64_t lo[4], hi[4];
+};
+template <int OFF>
+DEVINLINE VFrag read_v(const unsigned (&a)[4]) {
+  VFrag f;
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\t"
+      "ds_read_b64_tr_b16 %4, %8 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %1, %9\n\t"
+      "ds_read_b64_tr_b16 %5, %9 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %2, %10\n\t"
+      "ds_read_b64_tr_b16 %6, %10 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %3, %11\n\t"
+      "ds_read_b64_tr_b16 %7, %11 offset:%12\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(f.lo[0]), "=&v"(f.lo[1]), "=&v"(f.lo[2]), "=&v"(f.lo[3]),
+        "=&v"(f.hi[0]), "=&v"(f.hi[1]), "=&v"(f.hi[2]), "=&v"(f.hi[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "n"(OFF)
+      : "memory");
+  return f;
+}
+
+template <int N>
+DEVINLINE void waitcnt_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// out layout when SPLIT_MODE: partial [B, Hq, n_split, D] float, ml [B, Hq,
+// n_split, 2] float (m in log2 units, l); else bf16 out directly.
+// PAGED: k_cache/v_cache are page pools [n_pages, Hkv, 128, D] and
+// block_table [B, bt_stride] maps position/128 -> page id.
 template <int D, int SPLIT_MODE, int PAGED>
-__global__ __launch_bounds__(BLOCK) void decode_attn_mfma_kernel(
+__global__ __launch_bounds__(NWAVE * 64) void decode_attn_mfma_kernel(
     const bf16* __restrict__ q,        // [B, Hq, D]
     const bf16* __restrict__ k_cache,  // [B, Hkv, Smax, D] (or pool)
     const bf16* __restrict__ v_cache,
     const int* __restrict__ seq_lens,  // [B]
     const int* __restrict__ block_table,
     bf16* __restrict__ out,            // [B, Hq, D]
-    float* __restrict__ partial,       // [B, Hq, SPLIT, D]
-    float* __restrict__ partial_ml,    // [B, Hq, SPLIT, 2]
+    float* __restrict__ partial,
+    float* __restrict__ partial_ml,
     int Hq, int Hkv, int Smax, float scale, int n_split, int bt_stride,
     int per_row) {
   constexpr int KCH = D / 32;        // MFMA k-chunks for QK^T
-  constexpr int NS = D / 16;         // PV output col tiles
-  const int b = blockIdx.x;
-  const int hkv = blockIdx.y;
-  const int split = blockIdx.z;
-  const int G = Hq / Hkv;
-  const int h0 = hkv * G;
+  constexpr int NV = D / 16;         // 16-column tiles of V
+  constexpr int SL = D / 8, RPC = 64 / SL;   // slots per row, rows per copy
+  constexpr int CP = KT / RPC;               // copies per operand and tile
+  const int b = blockIdx.x, hkv = blockIdx.y, split = blockIdx.z;
+  const int G = Hq / Hkv, h0 = hkv * G;
   const int L = seq_lens[b];
 
-  // per_row: this ROW's split count comes from its own length (batch
-  // composition must not change a row's accumulation — exact-greedy
-  // guarantee); the launch z-width n_split is a host-side upper bound
-  // and surplus blocks exit.
+  // per_row: this ROW's slices come from its own length (batch composition
+  // must not change a row's accumulation — exact-greedy guarantee); the
+  // launch z-width n_split is a host-side upper bound, surplus blocks exit.
   const int ns_row = per_row ? tl_split_for_len(L) : n_split;
   if (split >= ns_row) return;
-
-  // this split's key range
-  const int per_split = (L + ns_row - 1) / ns_row;
+  const int per_split = (L + ns_row * KT - 1) / (ns_row * KT) * KT;
   const int k_begin = split * per_split;
   const int k_end = min(L, k_begin + per_split);
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int col = lane & 15;         // key-in-tile / head-col
-  const int quad = lane >> 4;        // 0..3
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, quad = lane >> 4;
 
-  // V as row-major [32 keys][16 dv] panels per (wave, dv-16-chunk): b128
-  // staging writes + ds_read_b64_tr_b16 fragment reads (no scatter
-  // transpose). Rows 16..31 stay zero — they feed the K=32 PV MFMA's
-  // upper half, so the quad<2 zero-branch disappears. Same for the upper
-  // half of the P tile.
-  constexpr int PSTRIDE = 32 * 16 + 8;
-  __shared__ bf16 v_pan[NWAVE * (D / 16) * PSTRIDE];
-  __shared__ bf16 p_lds[NWAVE][16][32 + 8];
-  __shared__ float red_m[NWAVE][16], red_l[NWAVE][16];
-  __shared__ float red_o[NWAVE][16][D];
+  __shared__ union alignas(16) {
+    bf16 buf[NWAVE][2][2][KT][D];            // [wave][buffer][k|v]
+    struct {
+      float o[NWAVE][16][D + 4];
+      float m[NWAVE][16], l[NWAVE][16];
+    } red;
+  } lds;
 
-  // one-time zero of the never-written upper halves
-  for (int i = threadIdx.x; i < NWAVE * (D / 16); i += BLOCK) {
-    for (int e = 0; e < 16 * 16; ++e)
-      v_pan[i * PSTRIDE + 16 * 16 + e] = f2bf(0.f);
-  }
-  for (int i = threadIdx.x; i < NWAVE * 16; i += BLOCK) {
-    for (int e = 16; e < 32; ++e) p_lds[i / 16][i % 16][e] = f2bf(0.f);
-  }
-  __syncthreads();
-
-  const bf16* kbase = k_cache + ((int64_t)b * Hkv + hkv) * Smax * D;
-  const bf16* vbase = v_cache + ((int64_t)b * Hkv + hkv) * Smax * D;
-
-  // ---- A fragments: q for this head group; rows >= G zeroed ----
-  bf16x8_t afrag[KCH];
+  // B operand: q of head col (zero past G), scale in exp2 units
+  bf16x8_t qf[KCH];
   {
-    const bool valid = col < G;
-    const bf16* qrow = q + ((int64_t)b * Hq + h0 + (valid ? col : 0)) * D;
+    const bf16* qrow =
+        q + ((int64_t)b * Hq + h0 + (col < G ? col : 0)) * D + quad * 8;
 #pragma unroll
     for (int c = 0; c < KCH; ++c) {
-      bf16x8_t f = *reinterpret_cast<const bf16x8_t*>(
-          qrow + c * 32 + quad * 8);
-      if (!valid)
+      qf[c] = *reinterpret_cast<const bf16x8_t*>(qrow + c * 32);
+      if (col >= G)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = (__bf16)0.f;
-      afrag[c] = f;
+        for (int j = 0; j < 8; ++j) qf[c][j] = (__bf16)0.f;
     }
   }
-
-  float m_run[4], l_run[4];
-  f32x4 oacc[NS];
+  float c2 = scale * LOG2E;
+  if (c2 < 0.f) {                            // exact: flip the query's sign
+    c2 = -c2;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) { m_run[r] = -1e30f; l_run[r] = 0.f; }
+    for (int c = 0; c < KCH; ++c)
 #pragma unroll
-  for (int n = 0; n < NS; ++n) oacc[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 8; ++j) qf[c][j] = -qf[c][j];
+  }
+  c2 = fmaxf(c2, 1e-30f);
 
-  // ---- main loop: each wave takes every NWAVE'th 16-key tile ----
-  for (int t0 = k_begin + wave * KT; t0 < k_end; t0 += NWAVE * KT) {
-    const int key = t0 + col;
-    const bool kv_ok = key < k_end;
-    const int safe_key = kv_ok ? key : (k_end - 1);
+  // pages of this slice: lane i holds the i-th of 64 (8192 keys) at a time
+  int pages = 0, page0 = k_begin >> 7;
+  auto load_pages = [&]() {
+    if (PAGED && k_begin < k_end)
+      pages = block_table[b * bt_stride +
+                          min(page0 + lane, (k_end - 1) >> 7)];
+  };
+  load_pages();
 
-    // B fragments straight from global K + stage V transposed into LDS
-    f32x4 sacc = (f32x4){0.f, 0.f, 0.f, 0.f};
-    {
-      const bf16 *krow, *vrow;
-      if (PAGED) {
-        const int page = block_table[b * bt_stride + (safe_key >> 7)];
-        const int64_t off =
-            (((int64_t)page * Hkv + hkv) * 128 + (safe_key & 127)) * D;
-        krow = k_cache + off;
-        vrow = v_cache + off;
-      } else {
-        krow = kbase + (int64_t)safe_key * D;
-        vrow = vbase + (int64_t)safe_key * D;
+  const int crow = lane / SL, cslot = lane % SL;
+  int koff[CP], voff[CP];
+#pragma unroll
+  for (int i = 0; i < CP; ++i) {
+    const int r = i * RPC + crow;
+    koff[i] = (cslot ^ k_perm<D>(r)) * 8;
+    voff[i] = (cslot ^ v_perm<D>(r)) * 8;
+  }
+  auto copy = [&](int bufi, int t0) {
+    int64_t base;
+    if (PAGED) {
+      if ((t0 >> 7) - page0 >= 64) {
+        page0 += 64;
+        load_pages();
       }
+      const int page = __builtin_amdgcn_readlane(pages, (t0 >> 7) - page0);
+      base = (((int64_t)page * Hkv + hkv) * 128 + (t0 & 127)) * D;
+    } else {
+      base = (((int64_t)b * Hkv + hkv) * Smax + t0) * D;
+    }
+    const bf16* kp = k_cache + base;
+    const bf16* vp = v_cache + base;
+    const int last = k_end - 1 - t0;         // keys past the end repeat it
+#pragma unroll
+    for (int i = 0; i < CP; ++i) {
+      const int ro = min(i * RPC + crow, last) * D;
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(kp + ro + koff[i]),
+          (__attribute__((address_space(3))) void*)(
+              &lds.buf[wave][bufi][0][i * RPC][0]),
+          16, 0, 0);
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(vp + ro + voff[i]),
+          (__attribute__((address_space(3))) void*)(
+              &lds.buf[wave][bufi][1][i * RPC][0]),
+          16, 0, 0);
+    }
+  };
+
+  // V^T reads: rows 4 quad + (lane >> 2) & 3 (and 16 on), columns 16 n
+  unsigned vaddr[NV];
+  {
+    const int r = quad * 4 + ((lane >> 2) & 3);
+    const unsigned base =
+        (unsigned)(uintptr_t)(&lds.buf[wave][0][1][0][0]) + r * D * 2 +
+        (lane & 1) * 8;
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      vaddr[n] = base + (((n * 2 + ((lane & 3) >> 1)) ^ v_perm<D>(r)) * 16);
+  }
+
+  float m_run = -1e30f, l_run = 0.f;         // log2 units; l of this lane
+  f32x4 o[NV];
+#pragma unroll
+  for (int n = 0; n < NV; ++n) o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  // ---- each wave takes every NWAVE'th tile ----
+  if (k_begin + wave * KT < k_end) copy(0, k_begin + wave * KT);
+  int buf = 0;
+  for (int t0 = k_begin + wave * KT; t0 < k_end; t0 += NWAVE * KT) {
+    const int next = t0 + NWAVE * KT;
+    if (next < k_end) {
+      copy(buf ^ 1, next);
+      waitcnt_vm<2 * CP>();
+    } else {
+      waitcnt_vm<0>();
+    }
+    f32x4 s[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      s[h] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int c = 0; c < KCH; ++c) {
-        bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(
-            krow + c * 32 + quad * 8);
-        sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag[c], kf, sacc,
-                                                       0, 0, 0);
-        // V: same addressing; b128 write into the (wave, dv-chunk) panel
-        bf16x8_t vf = *reinterpret_cast<const bf16x8_t*>(
-            vrow + c * 32 + quad * 8);
-        const int d0 = c * 32 + quad * 8;
-        const int pan = wave * (D / 16) + (d0 >> 4);
-        *reinterpret_cast<bf16x8_t*>(
-            &v_pan[pan * PSTRIDE + col * 16 + (d0 & 15)]) = vf;
+        const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(
+            &lds.buf[wave][buf][0][h * 16 + col]
+                    [((c * 4 + quad) ^ k_perm<D>(col)) * 8]);
+        s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[c], s[h], 0, 0,
+                                                       0);
       }
     }
-
-    // ---- online softmax on the 16-key score tile ----
-    // lane holds S[row=quad*4+r][col] in sacc[r]; per-ROW max (a shared
-    // 4-row max underflows exp when head score ranges differ by >88)
-    float p[4], row_max[4];
+    if (t0 + KT > k_end) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      sacc[r] = kv_ok ? sacc[r] * scale : -1e30f;
-      row_max[r] = sacc[r];
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (t0 + h * 16 + quad * 4 + r >= k_end) s[h][r] = -INFINITY;
     }
+    float mx = s[0][0];
 #pragma unroll
-    for (int off = 1; off < 16; off <<= 1)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        row_max[r] = fmaxf(row_max[r], __shfl_xor(row_max[r], off,
-                                                  WAVE_SIZE));
-    float m_new[4], alpha[4], psum[4];
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[h][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE_SIZE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE_SIZE)) * c2;
+    // the reference maximum moves only when it is exceeded by 2^8 (a
+    // decision of the head's own lanes): P and the sums stay far inside fp32
+    const bool up = mx > m_run + 8.f;
+    if (__any(up)) {
+      const float alpha = up ? __builtin_amdgcn_exp2f(m_run - mx) : 1.f;
+      m_run = up ? mx : m_run;
+      l_run *= alpha;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      m_new[r] = fmaxf(m_run[r], row_max[r]);
-      alpha[r] = __expf(m_run[r] - m_new[r]);
-      p[r] = (kv_ok) ? __expf(sacc[r] - m_new[r]) : 0.f;
-      psum[r] = p[r];
-      m_run[r] = m_new[r];
+      for (int n = 0; n < NV; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[n][r] *= alpha;
     }
+    bf16x8_t p;
+    float ps = 0.f;
 #pragma unroll
-    for (int off = 1; off < 16; off <<= 1)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        psum[r] += __shfl_xor(psum[r], off, WAVE_SIZE);
+      for (int r = 0; r < 4; ++r) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(s[h][r], c2, -m_run));
+        ps += e;
+        p[h * 4 + r] = (__bf16)e;
+      }
+    l_run += ps;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) l_run[r] = l_run[r] * alpha[r] + psum[r];
-
-    // P -> LDS (C-layout write), then A-fragment read. NO barriers here:
-    // each wave owns its own LDS slabs ([wave] index) and same-wave
-    // ds_write -> ds_read ordering is enforced by lgkmcnt; a block-wide
-    // barrier would deadlock (waves run different trip counts).
+    for (int g = 0; g < NV / 4; ++g) {
+      unsigned a[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      p_lds[wave][quad * 4 + r][col] = f2bf(p[r]);
-    // rescale O accumulators by alpha (row = quad*4+r)
+      for (int n = 0; n < 4; ++n) a[n] = vaddr[g * 4 + n] + buf * (2 * KT * D * 2);
+      const VFrag f = read_v<16 * D * 2>(a);
 #pragma unroll
-    for (int n = 0; n < NS; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) oacc[n][r] *= alpha[r];
-
-    // ---- PV: K=32 MFMA; keys 16..31 are the pre-zeroed halves ----
-    bf16x8_t pa = *reinterpret_cast<const bf16x8_t*>(
-        &p_lds[wave][col][quad * 8]);
-#pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      const unsigned pan_base = (unsigned)(uintptr_t)(
-          &v_pan[(wave * (D / 16) + n) * PSTRIDE]);
-      bf16x8_t vb = (bf16x8_t)ds_read_tr16_frag(
-          tr16_frag_addr(pan_base, lane));
-      oacc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vb, oacc[n],
-                                                        0, 0, 0);
+      for (int n = 0; n < 4; ++n) {
+        const uint64_t w[2] = {f.lo[n], f.hi[n]};
+        bf16x8_t vf;
+        __builtin_memcpy(&vf, w, 16);
+        o[g * 4 + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            vf, p, o[g * 4 + n], 0, 0, 0);
+      }
     }
+    buf ^= 1;                // read_v has waited for all reads of this buffer
   }
 
-  // ---- wave partials -> LDS ----
-  // lane holds O[row=quad*4+r][col=n*16+col]; every 16-lane group holds the
-  // full row set, so groups 1..3 duplicate group 0 -> write from quad 0..3
-  // cover distinct (row, col) pairs already: row=quad*4+r col covers only
-  // cols where lane&15 == col. Write all lanes (distinct rows per quad).
+  // ---- wave partials -> LDS: lane has columns 16 n + 4 quad + r of head col
+  l_run += __shfl_xor(l_run, 16, WAVE_SIZE);
+  l_run += __shfl_xor(l_run, 32, WAVE_SIZE);
+  __syncthreads();                           // all buffers are free
 #pragma unroll
-  for (int n = 0; n < NS; ++n)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      red_o[wave][quad * 4 + r][n * 16 + col] = oacc[n][r];
-  if (col == 0) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      red_m[wave][quad * 4 + r] = m_run[r];
-      red_l[wave][quad * 4 + r] = l_run[r];
-    }
+  for (int n = 0; n < NV; ++n)
+    *reinterpret_cast<f32x4*>(&lds.red.o[wave][col][n * 16 + quad * 4]) = o[n];
+  if (quad == 0) {
+    lds.red.m[wave][col] = m_run;
+    lds.red.l[wave][col] = l_run;
   }
   __syncthreads();
 
   // ---- final merge across waves; write out ----
-  const int g_count = min(G, 16);
-  for (int i = threadIdx.x; i < g_count * D; i += BLOCK) {
+  for (int i = threadIdx.x; i < G * D; i += NWAVE * 64) {
     const int g = i / D, d = i - g * D;
-    float m_tot = -1e30f;
+    float m_tot = lds.red.m[0][g];
 #pragma unroll
-    for (int w = 0; w < NWAVE; ++w) m_tot = fmaxf(m_tot, red_m[w][g]);
-    float l_tot = 0.f, o = 0.f;
+    for (int w = 1; w < NWAVE; ++w) m_tot = fmaxf(m_tot, lds.red.m[w][g]);
+    float l_tot = 0.f, acc = 0.f;
 #pragma unroll
     for (int w = 0; w < NWAVE; ++w) {
-      const float f = __expf(red_m[w][g] - m_tot);
-      l_tot += red_l[w][g] * f;
-      o += red_o[w][g][d] * f;
+      const float f = __builtin_amdgcn_exp2f(lds.red.m[w][g] - m_tot);
+      l_tot += lds.red.l[w][g] * f;
+      acc += lds.red.o[w][g][d] * f;
     }
     if (SPLIT_MODE) {
       const int64_t base = (((int64_t)b * Hq + h0 + g) * n_split + split);
-      partial[base * D + d] = o;
+      partial[base * D + d] = acc;
       if (d == 0) {
         partial_ml[base * 2] = m_tot;
         partial_ml[base * 2 + 1] = l_tot;
       }
     } else {
       out[((int64_t)b * Hq + h0 + g) * D + d] =
-          f2bf(o / fmaxf(l_tot, 1e-30f));
+          f2bf(acc / fmaxf(l_tot, 1e-30f));
     }
   }
 }
@@ -282,7 +349,7 @@ __global__ __launch_bounds__(128) void decode_attn_combine_kernel(
   for (int s = 0; s < ns_row; ++s) m_tot = fmaxf(m_tot, sm[s]);
   float l_tot = 0.f, o = 0.f;
   for (int s = 0; s < ns_row; ++s) {
-    const float f = __expf(sm[s] - m_tot);
+    const float f = __builtin_amdgcn_exp2f(sm[s] - m_tot);
     l_tot += sl[s] * f;
     o += partial[((int64_t)bh * n_split + s) * D + d] * f;
   }
@@ -301,7 +368,7 @@ void tl_decode_attn_mfma(const void* q, const void* k_cache,
                          void* partial, void* partial_ml, int B, int Hq,
                          int Hkv, int Smax, int D, float scale, int n_split,
                          int bt_stride, int per_row, hipStream_t stream) {
-  dim3 grid(B, Hkv, n_split), block(BLOCK);
+  dim3 grid(B, Hkv, n_split), block(NWAVE * 64);
 #define LAUNCH(DD, SM, PG)                                                   \
   hipLaunchKernelGGL((decode_attn_mfma_kernel<DD, SM, PG>), grid, block, 0,  \
                      stream, (const bf16*)q, (const bf16*)k_cache,           \

@@ -359,6 +359,45 @@ def test_tl_gemm(M, N, K, bias):
     torch.testing.assert_close(out.float(), ref, atol=5e-2, rtol=5e-2)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,lens,ns", [
+    (16, 1, 128, [1, 31, 32, 33], 0), (7, 1, 64, [127, 128, 129, 200], 0),
+    (8, 2, 64, [1, 300, 5, 257], 3),         # slices without keys
+    (4, 4, 128, [1024, 1025, 2049, 4097], 0),
+    (8, 2, 128, [8320, 8193], 1),            # one slice over 64 pages
+    (28, 4, 128, [20000, 3], 0),
+])
+@pytest.mark.parametrize("scale", [0.1, -0.1])
+def test_decode_attn_edges(Hq, Hkv, D, lens, ns, scale):
+    """Tile, slice and page edges against fp64, contiguous and paged with the
+    same bits. Inputs and P are rounded to bf16 (2^-9 relative): the 2-norm
+    error stays under 4e-3. Keys past a row's end are NaN and not seen."""
+    ops = _ext()
+    torch.manual_seed(len(lens) + D)
+    B, S = len(lens), (max(lens) + 127) // 128 * 128
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    q, k, v = mk(B, Hq, D), mk(B, Hkv, S, D), mk(B, Hkv, S, D)
+    want = []
+    for b, n in enumerate(lens):
+        kb, vb = (t[b, :, :n].double().repeat_interleave(Hq // Hkv, 0)
+                  for t in (k, v))
+        z = (q[b].double()[:, None] @ kb.transpose(1, 2)) * scale
+        want.append((z.softmax(-1) @ vb)[:, 0])
+        k[b, :, n:], v[b, :, n:] = math.nan, math.nan
+    want = torch.stack(want)
+    L = torch.tensor(lens, device=DEV, dtype=torch.int32)
+    out = ops.attention_decode(q, k, v, L, scale=scale, n_split=ns)
+    err = (out.double() - want).norm() / want.norm()
+    assert err < 4e-3, float(err)
+    table = torch.randperm(B * S // 128, device=DEV).int().view(B, -1)
+    pk, pv = mk(B * S // 128, Hkv, 128, D), mk(B * S // 128, Hkv, 128, D)
+    for t, pool in ((k, pk), (v, pv)):
+        pool[table.long().view(-1)] = t.view(B, Hkv, -1, 128, D).transpose(
+            1, 2).reshape(-1, Hkv, 128, D)
+    got = ops.attention_decode(q, pk, pv, L, scale=scale, n_split=ns,
+                               block_table=table)
+    assert torch.equal(got, out)
+
+
 @pytest.mark.parametrize("N,K", [
     (64, 32), (128, 160), (320, 544), (64, 2080),      # k remainders, 4 cuts
     (8192, 800), (16384, 288), (65600, 96),            # 2 cuts, none, wide
