@@ -133,6 +133,14 @@ class Attention(nn.Module):
         qkv = self.qkv_proj(x)
         flat_pos = positions.reshape(-1)
 
+        if training and not self.use_qk_norm and qkv.is_cuda:
+            q, k, v = ops.rope_rows(qkv.view(B * S, -1), flat_pos,
+                                    self.inv_freq, self.n_heads, self.n_kv)
+            out = ops.attention_train(q.view(B, S, self.n_heads, -1),
+                                      k.view(B, S, self.n_kv, -1),
+                                      v.view(B, S, self.n_kv, -1),
+                                      causal=True, scale=self.scale)
+            return self.o_proj(out.reshape(B, S, -1))
         if training or kv_cache is None:
             q, k, v = self._split_qkv(qkv, B, S)
             if self.use_qk_norm:
@@ -210,7 +218,8 @@ class MLP(nn.Module):
 
     def forward(self, x):
         gu = self.gate_up_proj(x)
-        if torch.is_grad_enabled() and gu.requires_grad:
+        if (torch.is_grad_enabled() and gu.requires_grad
+                and (not gu.is_cuda or self.inter % 8)):
             gate, up = gu.split([self.inter, self.inter], dim=-1)
             return self.down_proj(ops.swiglu(gate.contiguous(),
                                              up.contiguous()))

@@ -169,6 +169,39 @@ def apply_rope(q, k, positions, inv_freq):
     return _RopeFn.apply(q, k, positions, inv_freq)
 
 
+class _RopeRowsFn(torch.autograd.Function):
+    """RoPE between the fused projection's rows and q, k, v in one pass each
+    way (no split, clone or concatenation)."""
+
+    @staticmethod
+    def forward(ctx, qkv, positions, inv_freq, n_heads, n_kv):
+        positions = positions.int().contiguous()
+        inv_freq = inv_freq.float()
+        ctx.save_for_backward(positions, inv_freq)
+        return tuple(_require_ext().rope_split(qkv.contiguous(), positions,
+                                               inv_freq, n_heads, n_kv))
+
+    @staticmethod
+    def backward(ctx, dq, dk, dv):
+        positions, inv_freq = ctx.saved_tensors
+        return (_require_ext().rope_merge(
+            dq.contiguous(), dk.contiguous(), dv.contiguous(), positions,
+            inv_freq), None, None, None, None)
+
+
+def rope_rows(qkv: torch.Tensor, positions: torch.Tensor,
+              inv_freq: torch.Tensor, n_heads: int, n_kv: int):
+    """Training: rows [T, (n_heads + 2 n_kv) * D] of the fused projection to
+    q [T, n_heads, D] and k [T, n_kv, D], rotated, and v [T, n_kv, D]."""
+    D = 2 * inv_freq.numel()
+    if qkv.is_cuda and qkv.dtype == torch.bfloat16 and D % 16 == 0:
+        return _RopeRowsFn.apply(qkv, positions, inv_freq, n_heads, n_kv)
+    q, k, v = (t.reshape(t.shape[0], -1, D) for t in qkv.split(
+        [n_heads * D, n_kv * D, n_kv * D], dim=-1))
+    q, k = apply_rope(q, k, positions, inv_freq)
+    return q, k, v
+
+
 # ---------------------------------------------------------------------------
 # SwiGLU
 # ---------------------------------------------------------------------------
@@ -196,12 +229,28 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return _require_ext().swiglu_fwd(gate.contiguous(), up.contiguous())
 
 
+class _SwiGLUFusedFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, gate_up):
+        ctx.save_for_backward(gate_up)
+        return _require_ext().swiglu_fused(gate_up.contiguous())
+
+    @staticmethod
+    def backward(ctx, dout):
+        gate_up, = ctx.saved_tensors
+        return _require_ext().swiglu_fused_bwd(dout.contiguous(),
+                                               gate_up.contiguous())
+
+
 def swiglu_fused(gate_up: torch.Tensor) -> torch.Tensor:
     """silu(gu[..., :I]) * gu[..., I:] on the fused gate_up GEMM output
-    (inference path — avoids two .contiguous() splits)."""
+    (avoids two .contiguous() splits, and in training the concatenation of
+    their gradients)."""
     if not _on_gpu(gate_up):
         I = gate_up.shape[-1] // 2
         return ref.swiglu(gate_up[..., :I], gate_up[..., I:])
+    if torch.is_grad_enabled() and gate_up.requires_grad:
+        return _SwiGLUFusedFn.apply(gate_up)
     return _require_ext().swiglu_fused(gate_up.contiguous())
 
 

@@ -41,6 +41,11 @@ void tl_rope_append(const void* qkv, void* q_out, void* k_cache,
                     int D, int Smax, int bt_stride, hipStream_t stream);
 void tl_swiglu_fused(const void* gu, void* out, int64_t N, int I,
                      hipStream_t stream);
+void tl_swiglu_fused_bwd(const void* dout, const void* gu, void* dgu,
+                         int64_t N, int I, hipStream_t stream);
+void tl_rope_rows(void* qkv, void* q, void* k, void* v, const void* positions,
+                  const void* inv_freq, int64_t T, int Hq, int Hkv, int D,
+                  int bwd, hipStream_t stream);
 void tl_decode_attn_mfma(const void* q, const void* k_cache,
                          const void* v_cache, const void* seq_lens,
                          const void* block_table, void* out,
@@ -415,6 +420,60 @@ Tensor swiglu_fused(Tensor gu) {
   return out;
 }
 
+Tensor swiglu_fused_bwd(Tensor dout, Tensor gu) {
+  CHECK_IN(dout, torch::kBFloat16);
+  CHECK_IN(gu, torch::kBFloat16);
+  const int64_t I2 = gu.size(-1);
+  TORCH_CHECK(I2 % 16 == 0 && dout.numel() * 2 == gu.numel() &&
+                  dout.size(-1) * 2 == I2,
+              "dout must be half as wide as gate_up, a multiple of 8");
+  auto dgu = torch::empty_like(gu);
+  tl_swiglu_fused_bwd(dout.data_ptr(), gu.data_ptr(), dgu.data_ptr(),
+                      gu.numel() / std::max<int64_t>(I2, 1), (int)(I2 / 2),
+                      cur_stream());
+  return dgu;
+}
+
+// fused projection rows [T, (Hq + 2 Hkv) D] -> rotated q, k, and v
+std::vector<Tensor> rope_split(Tensor qkv, Tensor positions, Tensor inv_freq,
+                               int64_t Hq, int64_t Hkv) {
+  CHECK_IN(qkv, torch::kBFloat16);
+  CHECK_IN(positions, torch::kInt);
+  CHECK_IN(inv_freq, torch::kFloat);
+  const int64_t T = qkv.size(0), D = inv_freq.numel() * 2;
+  TORCH_CHECK(qkv.dim() == 2 && qkv.size(1) == (Hq + 2 * Hkv) * D &&
+                  D % 16 == 0 && positions.numel() == T,
+              "qkv width mismatch");
+  auto q = torch::empty({T, Hq, D}, qkv.options());
+  auto k = torch::empty({T, Hkv, D}, qkv.options());
+  auto v = torch::empty_like(k);
+  tl_rope_rows(qkv.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+               positions.data_ptr(), inv_freq.data_ptr(), T, (int)Hq,
+               (int)Hkv, (int)D, 0, cur_stream());
+  return {q, k, v};
+}
+
+// its backward
+Tensor rope_merge(Tensor dq, Tensor dk, Tensor dv, Tensor positions,
+                  Tensor inv_freq) {
+  CHECK_IN(dq, torch::kBFloat16);
+  CHECK_IN(dk, torch::kBFloat16);
+  CHECK_IN(dv, torch::kBFloat16);
+  CHECK_IN(positions, torch::kInt);
+  CHECK_IN(inv_freq, torch::kFloat);
+  const int64_t T = dq.size(0), Hq = dq.size(1), Hkv = dk.size(1);
+  const int64_t D = inv_freq.numel() * 2;
+  TORCH_CHECK(dq.dim() == 3 && dq.size(2) == D && D % 16 == 0 &&
+                  dk.size(0) == T && dk.size(2) == D &&
+                  dv.sizes() == dk.sizes() && positions.numel() == T,
+              "gradient shapes mismatch");
+  auto out = torch::empty({T, (Hq + 2 * Hkv) * D}, dq.options());
+  tl_rope_rows(out.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+               positions.data_ptr(), inv_freq.data_ptr(), T, (int)Hq,
+               (int)Hkv, (int)D, 1, cur_stream());
+  return out;
+}
+
 // Split-K policy SHARED by the streaming (M<=64) and tiled (M>64) GEMM
 // kernels. It depends only on (N, K) — never M — so a row's accumulation
 // (split boundaries + s-ordered reduce) is bitwise identical at every M:
@@ -545,6 +604,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
   mod.def("swiglu_fwd", &swiglu_fwd, "silu(gate)*up");
   mod.def("swiglu_bwd", &swiglu_bwd, "SwiGLU bwd");
   mod.def("adamw_", &adamw_, "fused AdamW step");
+  mod.def("swiglu_fused_bwd", &swiglu_fused_bwd,
+          "gradient of swiglu_fused as one tensor");
+  mod.def("rope_split", &rope_split,
+          "fused projection rows to rotated q, k, and v");
+  mod.def("rope_merge", &rope_merge,
+          "gradients of q, k, v rotated back into projection rows");
   mod.def("decode_attn", &decode_attn, "GQA decode attention over KV cache");
   mod.def("prefill_attn", &prefill_attn, "causal GQA prefill attention");
   mod.def("sample_tokens", &sample_tokens,

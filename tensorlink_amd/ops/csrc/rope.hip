@@ -44,9 +44,61 @@ __global__ __launch_bounds__(BLOCK) void rope_kernel(
   }
 }
 
+// Training, straight from and to the fused projection's rows [T, (Hq + 2 Hkv)
+// * D]. BWD 0: q and k rotated, and v, as tensors of their own. BWD 1: their
+// gradients rotated back into one gradient row. Eight elements of either half
+// of a head per thread; the angle is that of rope_kernel.
+template <int BWD>
+__global__ __launch_bounds__(BLOCK) void rope_rows_kernel(
+    bf16* __restrict__ qkv, bf16* __restrict__ q, bf16* __restrict__ k,
+    bf16* __restrict__ v, const int* __restrict__ positions,
+    const float* __restrict__ inv_freq, int Hq, int Hkv, int D) {
+  const int64_t token = blockIdx.x;
+  const float pos = (float)positions[token];
+  const int D2 = D / 2, C = D2 / 8, H = Hq + 2 * Hkv;
+  bf16* row = qkv + token * H * D;
+  for (int i = threadIdx.x; i < H * C; i += BLOCK) {
+    const int h = i / C, d = (i - h * C) * 8;
+    bf16* part = h < Hq ? q + (token * Hq + h) * D
+                 : h < Hq + Hkv ? k + (token * Hkv + h - Hq) * D
+                                : v + (token * Hkv + h - Hq - Hkv) * D;
+    const bf16* src = BWD ? part : row + h * D;
+    bf16* dst = BWD ? row + h * D : part;
+    bf16x8 a = *reinterpret_cast<const bf16x8*>(src + d);
+    bf16x8 b = *reinterpret_cast<const bf16x8*>(src + d + D2);
+    if (h < Hq + Hkv) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float c, s;
+        __sincosf(pos * inv_freq[d + j], &s, &c);
+        if (BWD) s = -s;
+        const float x1 = bf2f(a.v[j]), x2 = bf2f(b.v[j]);
+        a.v[j] = f2bf(x1 * c - x2 * s);
+        b.v[j] = f2bf(x2 * c + x1 * s);
+      }
+    }
+    *reinterpret_cast<bf16x8*>(dst + d) = a;
+    *reinterpret_cast<bf16x8*>(dst + d + D2) = b;
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+// D a multiple of 16
+void tl_rope_rows(void* qkv, void* q, void* k, void* v, const void* positions,
+                  const void* inv_freq, int64_t T, int Hq, int Hkv, int D,
+                  int bwd, hipStream_t stream) {
+  if (T <= 0) return;
+#define TL_RR(B)                                                             \
+  hipLaunchKernelGGL(rope_rows_kernel<B>, dim3((uint32_t)T), dim3(BLOCK), 0, \
+                     stream, (bf16*)qkv, (bf16*)q, (bf16*)k, (bf16*)v,       \
+                     (const int*)positions, (const float*)inv_freq, Hq, Hkv, \
+                     D)
+  if (bwd) TL_RR(1); else TL_RR(0);
+#undef TL_RR
+}
 
 void tl_rope(void* q, void* k, const void* positions, const void* inv_freq,
              int64_t T, int Hq, int Hkv, int D, float sign,

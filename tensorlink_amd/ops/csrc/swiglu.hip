@@ -44,6 +44,13 @@ __global__ __launch_bounds__(BLOCK) void swiglu_fused_kernel(
   *reinterpret_cast<bf16x8*>(out + r * I + c) = o;
 }
 
+DEVINLINE void swiglu_grad(float dO, float g, float u, bf16& dg, bf16& du) {
+  const float sig = 1.f / (1.f + __expf(-g));
+  const float dsilu = sig * (1.f + g * (1.f - sig));
+  dg = f2bf(dO * u * dsilu);
+  du = f2bf(dO * (g * sig));
+}
+
 __global__ __launch_bounds__(BLOCK) void swiglu_bwd_kernel(
     const bf16* __restrict__ dout, const bf16* __restrict__ gate,
     const bf16* __restrict__ up, bf16* __restrict__ dgate,
@@ -55,22 +62,44 @@ __global__ __launch_bounds__(BLOCK) void swiglu_bwd_kernel(
   bf16x8 u = reinterpret_cast<const bf16x8*>(up)[i];
   bf16x8 dg, du;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float gv = bf2f(g.v[j]);
-    const float sig = 1.f / (1.f + __expf(-gv));
-    const float si = gv * sig;
-    const float dsilu = sig * (1.f + gv * (1.f - sig));
-    const float dov = bf2f(dO.v[j]);
-    dg.v[j] = f2bf(dov * bf2f(u.v[j]) * dsilu);
-    du.v[j] = f2bf(dov * si);
-  }
+  for (int j = 0; j < 8; ++j)
+    swiglu_grad(bf2f(dO.v[j]), bf2f(g.v[j]), bf2f(u.v[j]), dg.v[j], du.v[j]);
   reinterpret_cast<bf16x8*>(dgate)[i] = dg;
   reinterpret_cast<bf16x8*>(dup)[i] = du;
+}
+
+// backward of swiglu_fused: gu [N, 2I], dout [N, I] -> dgu [N, 2I], so that
+// neither the halves of gu nor those of its gradient are copied
+__global__ __launch_bounds__(BLOCK) void swiglu_fused_bwd_kernel(
+    const bf16* __restrict__ dout, const bf16* __restrict__ gu,
+    bf16* __restrict__ dgu, int64_t N, int I) {
+  const int64_t i = ((int64_t)blockIdx.x * BLOCK + threadIdx.x) * 8;
+  if (i >= N * (int64_t)I) return;
+  const int64_t at = i / I * I + i;          // row * 2I + column
+  const bf16x8 dO = *reinterpret_cast<const bf16x8*>(dout + i);
+  const bf16x8 g = *reinterpret_cast<const bf16x8*>(gu + at);
+  const bf16x8 u = *reinterpret_cast<const bf16x8*>(gu + at + I);
+  bf16x8 dg, du;
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    swiglu_grad(bf2f(dO.v[j]), bf2f(g.v[j]), bf2f(u.v[j]), dg.v[j], du.v[j]);
+  *reinterpret_cast<bf16x8*>(dgu + at) = dg;
+  *reinterpret_cast<bf16x8*>(dgu + at + I) = du;
 }
 
 }  // namespace
 
 extern "C" {
+
+void tl_swiglu_fused_bwd(const void* dout, const void* gu, void* dgu,
+                         int64_t N, int I, hipStream_t stream) {
+  const int64_t work = N * (int64_t)I / 8;
+  if (work <= 0) return;
+  hipLaunchKernelGGL(swiglu_fused_bwd_kernel,
+                     dim3((uint32_t)((work + BLOCK - 1) / BLOCK)),
+                     dim3(BLOCK), 0, stream, (const bf16*)dout,
+                     (const bf16*)gu, (bf16*)dgu, N, I);
+}
 
 void tl_swiglu_fwd(const void* gate, const void* up, void* out, int64_t n,
                    hipStream_t stream) {

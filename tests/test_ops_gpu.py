@@ -236,6 +236,89 @@ def test_adamw_matches_torch():
                                rtol=2e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,off", [(1, 0), (7, 0), (8, 0), (2051, 0),
+                                   (2048, 1), (4099, 3)])
+def test_adamw_any_length_and_alignment(dtype, n, off):
+    """The vector kernel's remainder and the unaligned kernel give what fp64
+    gives: moments to fp32 rounding, weights to their own type's."""
+    ops = _ext()
+    torch.manual_seed(n)
+    mk = lambda d: torch.randn(n + off, device=DEV).to(d)[off:]
+    p, g, m, v = mk(dtype), mk(dtype), mk(torch.float32), \
+        mk(torch.float32).abs()
+    pd, gd, md, vd = (t.double() for t in (p, g, m, v))
+    md, vd = 0.9 * md + 0.1 * gd, 0.99 * vd + 0.01 * gd * gd
+    pd = pd * (1 - 1e-2 * 0.1) - 1e-2 * (md / (1 - 0.9 ** 3)) / (
+        (vd / (1 - 0.99 ** 3)).sqrt() + 1e-8)
+    ops.adamw_(p, g, m, v, lr=1e-2, beta1=0.9, beta2=0.99, eps=1e-8,
+               weight_decay=0.1, step=3)
+    torch.testing.assert_close(m.double(), md, atol=1e-6, rtol=1e-6)
+    torch.testing.assert_close(v.double(), vd, atol=1e-6, rtol=1e-6)
+    tol = 2 ** -8 if dtype == torch.bfloat16 else 1e-5
+    torch.testing.assert_close(p.double(), pd, atol=tol * 1e-2, rtol=tol)
+
+
+@pytest.mark.parametrize("N,H", [(1, 64), (5, 64), (33, 128), (700, 128),
+                                 (9, 256), (3, 512), (40, 520), (3, 3584)])
+def test_rmsnorm_widths(N, H):
+    """Rows of a few lanes and of a block, both directions, against fp64:
+    results are rounded to bf16 (2^-9), the 2-norm error stays under 4e-3."""
+    ops = _ext()
+    torch.manual_seed(N + H)
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    x, w, dy = mk(N, H), mk(H), mk(N, H)
+    xs, ws = x.clone().requires_grad_(True), w.clone().requires_grad_(True)
+    y = ops.rmsnorm(xs, ws, 1e-6)
+    y.backward(dy)
+    xd, wd = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    yd = xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + 1e-6) * wd
+    yd.backward(dy.double())
+    for a, b in ((y, yd), (xs.grad, xd.grad), (ws.grad, wd.grad)):
+        assert (a.double() - b).norm() / b.norm() < 4e-3
+    assert torch.equal(ops.rmsnorm(x, w, 1e-6), y)
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,D", [(1, 1, 1, 16), (5, 7, 1, 64),
+                                        (37, 4, 2, 128), (3, 28, 4, 80)])
+def test_rope_rows(T, Hq, Hkv, D):
+    """The same bits as the separate path in both directions."""
+    ops = _ext()
+    torch.manual_seed(T)
+    rows = torch.randn(T, (Hq + 2 * Hkv) * D, device=DEV,
+                       dtype=torch.bfloat16)
+    pos = torch.arange(100, 100 + T, device=DEV, dtype=torch.int32)
+    inv = 1e4 ** (-torch.arange(0, D, 2, device=DEV).float() / D)
+    a = rows.clone().requires_grad_(True)
+    b = rows.clone().requires_grad_(True)
+    got = ops.rope_rows(a, pos, inv, Hq, Hkv)
+    q, k, v = (t.reshape(T, -1, D) for t in
+               b.split([Hq * D, Hkv * D, Hkv * D], -1))
+    want = (*ops.apply_rope(q, k, pos, inv), v)
+    dy = [torch.randn_like(t) for t in want]
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
+    torch.autograd.backward(got, dy)
+    torch.autograd.backward(want, dy)
+    assert torch.equal(a.grad, b.grad)
+
+
+@pytest.mark.parametrize("N,I", [(1, 8), (3, 24), (65, 512), (7, 18944)])
+def test_swiglu_fused_backward(N, I):
+    """The same bits as from the split halves."""
+    ops = _ext()
+    torch.manual_seed(I)
+    gu = 3 * torch.randn(2, N, 2 * I, device=DEV, dtype=torch.bfloat16)
+    a, b = gu.clone().requires_grad_(True), gu.clone().requires_grad_(True)
+    y = ops.swiglu_fused(a)
+    g, u = b.split([I, I], -1)
+    z = ops.swiglu(g.contiguous(), u.contiguous())
+    dy = torch.randn_like(y)
+    y.backward(dy)
+    z.backward(dy)
+    assert torch.equal(y, z) and torch.equal(a.grad, b.grad)
+
+
 def test_decode_attn_softmax_stability():
     """Large score magnitudes must not overflow (online softmax)."""
     ops = _ext()
