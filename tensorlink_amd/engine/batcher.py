@@ -101,9 +101,6 @@ class _SlotView:
     def advance(self, n):
         pass   # slot lengths are tracked by the scheduler
 
-    def gather_contiguous(self, layer, S):
-        return PagedKVCache.gather_contiguous(self, layer, S)
-
     def append(self, layer, k_new, v_new, positions):
         return PagedKVCache.append(self, layer, k_new, v_new, positions)
 

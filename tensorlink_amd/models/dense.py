@@ -71,6 +71,30 @@ class TLLinear(nn.Linear):
         return ops.linear(x, self.weight, self.bias)
 
 
+def _unwatched(module: nn.Module) -> bool:
+    """Nobody sees this module's call: no hooks, no forward of its own."""
+    return not (module._forward_hooks or module._forward_pre_hooks
+                or "forward" in module.__dict__
+                or nn.modules.module._has_any_global_hook())
+
+
+def _serving(linear: nn.Module, x: torch.Tensor) -> bool:
+    """linear(x) is one product of the serving GEMM family and nothing else,
+    so that what follows may take its fp32 cuts of K as they are."""
+    return (type(linear) is TLLinear and _unwatched(linear)
+            and ops.serving_gemm(x, linear.weight))
+
+
+def cached_rows(kv_cache) -> int:
+    """Positions that a multi-token step finds in the cache: one for the
+    whole view, so rows have to agree (ragged multi-token work goes through
+    the decode path instead)."""
+    lens = kv_cache.seq_lens.tolist()
+    assert min(lens) == max(lens), \
+        "ragged cached prefill needs per-row q_off"
+    return lens[0]
+
+
 def compute_inv_freq(config: ModelConfig) -> torch.Tensor:
     """RoPE inverse frequencies, honoring HF rope_scaling. Implements
     the Llama-3.1 "llama3" spectrum scaling (long wavelengths divided by
@@ -127,11 +151,21 @@ class Attention(nn.Module):
 
     def forward(self, x: torch.Tensor, positions: torch.Tensor,
                 kv_cache: Optional[KVCache] = None, layer_idx: int = 0,
-                training: bool = False) -> torch.Tensor:
+                training: bool = False, q_off: Optional[int] = None
+                ) -> torch.Tensor:
+        return self.o_proj(self.mix(x, positions, kv_cache, layer_idx,
+                                    training, q_off))
+
+    def mix(self, x, positions, kv_cache=None, layer_idx=0, training=False,
+            q_off=None):
+        """All of it but the output projection. q_off: positions already in
+        the cache, where the caller has counted them (multi-token steps)."""
         B, S, H = x.shape
         eps = self.config.rms_norm_eps
-        qkv = self.qkv_proj(x)
         flat_pos = positions.reshape(-1)
+        if not training and kv_cache is not None:
+            return self._mix_cached(x, flat_pos, kv_cache, layer_idx, q_off)
+        qkv = self.qkv_proj(x)
 
         if training and not self.use_qk_norm and qkv.is_cuda:
             q, k, v = ops.rope_rows(qkv.view(B * S, -1), flat_pos,
@@ -140,71 +174,63 @@ class Attention(nn.Module):
                                       k.view(B, S, self.n_kv, -1),
                                       v.view(B, S, self.n_kv, -1),
                                       causal=True, scale=self.scale)
-            return self.o_proj(out.reshape(B, S, -1))
-        if training or kv_cache is None:
-            q, k, v = self._split_qkv(qkv, B, S)
-            if self.use_qk_norm:
-                q = ops.rmsnorm(q.contiguous(), self.q_norm.to(q.dtype), eps)
-                k = ops.rmsnorm(k.contiguous(), self.k_norm.to(k.dtype), eps)
-            if training:
-                q2, k2 = ops.apply_rope(q.reshape(B * S, self.n_heads, -1),
-                                        k.reshape(B * S, self.n_kv, -1),
-                                        flat_pos, self.inv_freq)
-                q = q2.view(B, S, self.n_heads, -1)
-                k = k2.view(B, S, self.n_kv, -1)
-                out = ops.attention_train(q, k, v, causal=True,
-                                          scale=self.scale)
-            else:
-                q = q.contiguous()
-                k = k.contiguous()
-                ops.apply_rope_(q.view(B * S, self.n_heads, -1),
-                                k.view(B * S, self.n_kv, -1), flat_pos,
-                                self.inv_freq)
-                out = ops.attention_prefill(q, k, v.contiguous(),
-                                            causal=True, scale=self.scale)
-            return self.o_proj(out.reshape(B, S, -1))
-
-        # inference with KV cache: fused rope+append straight off the
-        # fused-QKV rows (q comes back contiguous, k/v land in the cache;
-        # paged caches pass their block table through to the kernels)
-        table = getattr(kv_cache, "table", None)
+            return out.reshape(B, S, -1)
+        q, k, v = self._split_qkv(qkv, B, S)
         if self.use_qk_norm:
-            q, k, v = self._split_qkv(qkv, B, S)
             q = ops.rmsnorm(q.contiguous(), self.q_norm.to(q.dtype), eps)
             k = ops.rmsnorm(k.contiguous(), self.k_norm.to(k.dtype), eps)
-            qkv = torch.cat([q.reshape(B, S, -1), k.reshape(B, S, -1),
-                             v.reshape(B, S, -1)], dim=-1)
-        q = ops.rope_append_(qkv.reshape(B * S, -1), kv_cache.k[layer_idx],
-                             kv_cache.v[layer_idx], flat_pos, self.inv_freq,
-                             S, self.n_heads, self.n_kv, block_table=table)
+        if training:
+            q2, k2 = ops.apply_rope(q.reshape(B * S, self.n_heads, -1),
+                                    k.reshape(B * S, self.n_kv, -1),
+                                    flat_pos, self.inv_freq)
+            q = q2.view(B, S, self.n_heads, -1)
+            k = k2.view(B, S, self.n_kv, -1)
+            out = ops.attention_train(q, k, v, causal=True, scale=self.scale)
+        else:
+            q = q.contiguous()
+            k = k.contiguous()
+            ops.apply_rope_(q.view(B * S, self.n_heads, -1),
+                            k.view(B * S, self.n_kv, -1), flat_pos,
+                            self.inv_freq)
+            out = ops.attention_prefill(q, k, v.contiguous(), causal=True,
+                                        scale=self.scale)
+        return out.reshape(B, S, -1)
+
+    def _mix_cached(self, x, flat_pos, kv_cache, layer_idx, q_off):
+        """Inference with a KV cache: fused norm + rope + append straight off
+        the fused-QKV rows (q comes back contiguous, k/v land in the cache;
+        paged caches pass their block table through to the kernels)."""
+        B, S, _ = x.shape
+        table = getattr(kv_cache, "table", None)
+        k, v = kv_cache.k[layer_idx], kv_cache.v[layer_idx]
+        qw = self.q_norm.to(x.dtype) if self.use_qk_norm else None
+        kw = self.k_norm.to(x.dtype) if self.use_qk_norm else None
+        proj, eps = self.qkv_proj, self.config.rms_norm_eps
+        if _serving(proj, x) and (qw is None
+                                  or ops.head_norm_fits(self.head_dim)):
+            q = ops.linear_rope_append_(
+                x, proj.weight, proj.bias, k, v, flat_pos, self.inv_freq, S,
+                self.n_heads, self.n_kv, table, qw, kw, eps)
+        else:
+            q = ops.rope_append_(
+                proj(x).reshape(B * S, -1), k, v, flat_pos, self.inv_freq, S,
+                self.n_heads, self.n_kv, table, qw, kw, eps)
         q = q.view(B, S, self.n_heads, self.head_dim)
         if S == 1:
-            out = ops.attention_decode(
-                q, kv_cache.k[layer_idx], kv_cache.v[layer_idx],
-                kv_cache.seq_lens + 1, scale=self.scale, block_table=table)
+            out = ops.attention_decode(q, k, v, kv_cache.seq_lens,
+                                       scale=self.scale, block_table=table,
+                                       len_add=1)
         else:
-            # prefill with cache write; rotated k / raw v are read back from
-            # the cache. off > 0 = chunked prefill continuing an existing
-            # sequence (the chunk's queries sit at global rows off..off+S-1
-            # and attend to all off+S cached keys). A single q_off serves
-            # the whole view, so cached lengths must agree per row (ragged
-            # multi-token work goes through the decode path instead).
-            if B > 1:
-                assert int(kv_cache.seq_lens.min()) == \
-                    int(kv_cache.seq_lens.max()), \
-                    "ragged cached prefill needs per-row q_off"
-            off = int(kv_cache.seq_lens.max())
-            kv_len = off + S
-            if table is None:
-                k_attn = kv_cache.k[layer_idx][:, :, :kv_len].permute(
-                    0, 2, 1, 3).contiguous()
-                v_attn = kv_cache.v[layer_idx][:, :, :kv_len].permute(
-                    0, 2, 1, 3).contiguous()
-            else:
-                k_attn, v_attn = kv_cache.gather_contiguous(layer_idx, kv_len)
-            out = ops.attention_prefill(q, k_attn, v_attn, causal=True,
-                                        scale=self.scale, q_off=off)
-        return self.o_proj(out.reshape(B, S, -1))
+            # rotated k / raw v are read back from the cache. q_off > 0 =
+            # chunked prefill continuing an existing sequence (the chunk's
+            # queries sit at global rows q_off..q_off+S-1 and attend to all
+            # q_off+S cached keys).
+            if q_off is None:
+                q_off = cached_rows(kv_cache)
+            out = ops.attention_prefill_cache(q, k, v, q_off + S,
+                                              scale=self.scale,
+                                              block_table=table)
+        return out.reshape(B, S, -1)
 
 
 class MLP(nn.Module):
@@ -217,13 +243,16 @@ class MLP(nn.Module):
         self.down_proj = TLLinear(i, h, bias=False)
 
     def forward(self, x):
+        return self.down_proj(self.inner(x))
+
+    def inner(self, x):
+        """All of it but the down projection."""
         gu = self.gate_up_proj(x)
         if (torch.is_grad_enabled() and gu.requires_grad
                 and (not gu.is_cuda or self.inter % 8)):
             gate, up = gu.split([self.inter, self.inter], dim=-1)
-            return self.down_proj(ops.swiglu(gate.contiguous(),
-                                             up.contiguous()))
-        return self.down_proj(ops.swiglu_fused(gu))
+            return ops.swiglu(gate.contiguous(), up.contiguous())
+        return ops.swiglu_fused(gu)
 
 
 class MoEMLP(nn.Module):
@@ -325,7 +354,11 @@ class DecoderLayer(nn.Module):
         self.mlp = MoEMLP(config) if config.is_moe else MLP(config)
 
     def forward(self, hidden, positions, kv_cache=None, layer_idx=0,
-                training=False):
+                training=False, q_off=None, normed=None, next_norm=None):
+        """normed: this layer's input norm, where the layer below has taken
+        it already. next_norm: the weight of the norm that comes next; the
+        result is then (that norm of the layer's output, the output).
+        q_off: see Attention.mix. All three: inference on the GPU."""
         eps = self.config.rms_norm_eps
         w_in = self.input_layernorm.to(hidden.dtype)
         w_post = self.post_attention_layernorm.to(hidden.dtype)
@@ -337,10 +370,36 @@ class DecoderLayer(nn.Module):
             hidden = hidden + self.mlp(h)
             return hidden
         # inference: fused residual + norm (one HBM round trip)
-        h = ops.rmsnorm(hidden, w_in, eps)
-        attn_out = self.self_attn(h, positions, kv_cache, layer_idx, False)
-        h, hidden = ops.rmsnorm_residual(attn_out, hidden, w_post, eps)
-        return hidden + self.mlp(h)
+        h = normed if normed is not None else ops.rmsnorm(hidden, w_in, eps)
+        attn, mlp = self.self_attn, self.mlp
+        if (type(attn) is Attention and _unwatched(attn)
+                and ops.add_norm_fits(hidden)):
+            h = attn.mix(h, positions, kv_cache, layer_idx, False, q_off)
+            if _serving(attn.o_proj, h) and attn.o_proj.bias is None:
+                h, hidden = ops.linear_add_norm(
+                    h, attn.o_proj.weight, hidden, w_post, eps, False)
+            else:
+                h, hidden = ops.rmsnorm_residual(attn.o_proj(h), hidden,
+                                                 w_post, eps)
+        else:
+            h, hidden = ops.rmsnorm_residual(
+                attn(h, positions, kv_cache, layer_idx, False), hidden,
+                w_post, eps)
+        down = mlp.down_proj if type(mlp) is MLP else None
+        if next_norm is None and not ops.add_norm_fits(hidden):
+            return hidden + mlp(h)
+        if down is not None and _unwatched(mlp):
+            h = mlp.inner(h)
+            if _serving(down, h) and down.bias is None:
+                h, hidden = ops.linear_add_norm(h, down.weight, hidden,
+                                                next_norm, eps, True)
+                return hidden if next_norm is None else (h, hidden)
+            h = down(h)
+        else:
+            h = mlp(h)
+        if next_norm is None:
+            return hidden + h
+        return ops.add_norm(h, hidden, next_norm, eps)
 
 
 class StageModel(nn.Module):
@@ -388,9 +447,11 @@ class StageModel(nn.Module):
         w = self.embed_tokens.weight
         return self.embed_tokens(input_ids).to(w.dtype)
 
-    def head(self, hidden: torch.Tensor) -> torch.Tensor:
-        h = ops.rmsnorm(hidden, self.norm.to(hidden.dtype),
-                        self.config.rms_norm_eps)
+    def head(self, hidden: torch.Tensor,
+             normed: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """Logits; normed: the final norm of hidden, if it is there."""
+        h = normed if normed is not None else ops.rmsnorm(
+            hidden, self.norm.to(hidden.dtype), self.config.rms_norm_eps)
         if self.config.tie_word_embeddings and self.has_embedding:
             return h @ self.embed_tokens.weight.t()
         return self.lm_head(h)
@@ -405,6 +466,9 @@ class StageModel(nn.Module):
             hidden = hidden_or_ids
         ckpt = (training and getattr(self, "grad_checkpointing", False)
                 and torch.is_grad_enabled())
+        logits = self.has_head and return_logits
+        if not training and hidden.is_cuda and ops.add_norm_fits(hidden):
+            return self._serve(hidden, positions, kv_cache, logits)
         for i, layer in enumerate(self.layers):
             if ckpt:
                 # recompute the layer in backward instead of stashing
@@ -416,9 +480,35 @@ class StageModel(nn.Module):
                 hidden = layer(hidden, positions, kv_cache, i, training)
         if kv_cache is not None:
             kv_cache.advance(hidden.shape[1])
-        if self.has_head and return_logits:
-            return self.head(hidden)
-        return hidden
+        return self.head(hidden) if logits else hidden
+
+    def _serve(self, hidden, positions, kv_cache, logits):
+        """Inference on the GPU: a layer's last residual add takes the next
+        norm with it, and what is the same for all layers is done once."""
+        q_off = None
+        if kv_cache is not None:
+            positions = positions.int()
+            if hidden.shape[1] > 1 and self.layers:
+                q_off = cached_rows(kv_cache)
+        normed = None
+        plain = [type(m) is DecoderLayer and _unwatched(m)
+                 for m in self.layers]
+        for i, layer in enumerate(self.layers):
+            if not plain[i]:
+                hidden, normed = layer(hidden, positions, kv_cache, i), None
+                continue
+            nxt = None
+            if i + 1 < len(self.layers):
+                if plain[i + 1]:
+                    nxt = self.layers[i + 1].input_layernorm
+            elif logits:
+                nxt = self.norm
+            out = layer(hidden, positions, kv_cache, i, False, q_off, normed,
+                        None if nxt is None else nxt.to(hidden.dtype))
+            normed, hidden = out if nxt is not None else (None, out)
+        if kv_cache is not None:
+            kv_cache.advance(hidden.shape[1])
+        return self.head(hidden, normed) if logits else hidden
 
 
 def build_full_model(config: ModelConfig):

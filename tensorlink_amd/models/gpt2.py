@@ -69,23 +69,15 @@ class Gpt2Attention(nn.Module):
             if S == 1:
                 out = ops.attention_decode(
                     q, kv_cache.k[layer_idx], kv_cache.v[layer_idx],
-                    kv_cache.seq_lens + 1, scale=self.scale,
-                    block_table=table)
+                    kv_cache.seq_lens, scale=self.scale,
+                    block_table=table, len_add=1)
             else:
                 # prefill with cache; off > 0 = chunked continuation
                 # (same contract as models/dense.py Attention)
                 off = int(kv_cache.seq_lens.max())
-                kv_len = off + S
-                if table is None:
-                    k_attn = kv_cache.k[layer_idx][:, :, :kv_len].permute(
-                        0, 2, 1, 3).contiguous()
-                    v_attn = kv_cache.v[layer_idx][:, :, :kv_len].permute(
-                        0, 2, 1, 3).contiguous()
-                else:
-                    k_attn, v_attn = kv_cache.gather_contiguous(layer_idx,
-                                                                kv_len)
-                out = ops.attention_prefill(q, k_attn, v_attn, causal=True,
-                                            scale=self.scale, q_off=off)
+                out = ops.attention_prefill_cache(
+                    q, kv_cache.k[layer_idx], kv_cache.v[layer_idx], off + S,
+                    scale=self.scale, block_table=table)
         return self.c_proj(out.reshape(B, S, H))
 
 

@@ -4,7 +4,7 @@ The paged-KV decode kernel is the long-context story: instead of one
 contiguous [B, Hkv, Smax, D] slab per sequence, K/V
 live in a shared pool of 128-position pages and a per-sequence block table
 maps position/128 -> page id. The decode and rope+append kernels take the
-table (decode_attn_mfma.hip / rope_append.hip, PAGED variants), so
+table (decode_attn_mfma.hip, fused_rows.hip, prefill_attn.hip), so
 sequences only consume memory for pages they actually touch and a long
 context never needs a contiguous reservation.
 
@@ -68,18 +68,6 @@ class PagedKVCache:
             self.k[layer].dtype)
         self.v[layer][page, :, off] = v_new.reshape(B * S, H, D).to(
             self.v[layer].dtype)
-
-    def gather_contiguous(self, layer: int, S: int):
-        """Materialize the first S positions as [B, S, Hkv, D] (prefill
-        attention readback; once per request)."""
-        np = (S + PAGE - 1) // PAGE
-        idx = self.table[:, :np].long()                        # [B, np]
-        k = self.k[layer][idx]                                 # [B,np,H,PAGE,D]
-        v = self.v[layer][idx]
-        B, _, H, _, D = k.shape
-        k = k.permute(0, 1, 3, 2, 4).reshape(B, np * PAGE, H, D)
-        v = v.permute(0, 1, 3, 2, 4).reshape(B, np * PAGE, H, D)
-        return k[:, :S].contiguous(), v[:, :S].contiguous()
 
 
 class PageAllocator:

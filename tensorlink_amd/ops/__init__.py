@@ -107,22 +107,101 @@ def apply_rope_(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor,
     _require_ext().rope_(q, k, positions.int(), inv_freq.float(), sign)
 
 
+def add_norm_fits(x: torch.Tensor) -> bool:
+    """add_norm and linear_add_norm have no gradients and take bf16 rows of
+    whole 16-byte pieces that a block's registers hold."""
+    return (x.is_cuda and x.dtype == torch.bfloat16
+            and not torch.is_grad_enabled() and x.shape[-1] % 8 == 0
+            and x.shape[-1] <= 16384 and x.numel() > 0)
+
+
+def add_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
+             eps: float):
+    """r = x + residual as it is stored, y = RMSNorm(r) * weight: the end of
+    one layer and the first norm of the next (inference path).
+    Returns (y, r)."""
+    return _require_ext().add_norm(x.contiguous(), residual.contiguous(),
+                                   weight.contiguous(), eps, True)
+
+
+def linear_add_norm(x: torch.Tensor, weight: torch.Tensor,
+                    residual: torch.Tensor, norm: Optional[torch.Tensor],
+                    eps: float, rounded: bool):
+    """r = x @ weight^T + residual, y = RMSNorm(r) * norm, for a product that
+    serving_gemm() takes: the norm sums the cuts of K itself. rounded: it
+    sees r as it is stored, else the fp32 sum. Returns (y, r); norm None:
+    (None, r)."""
+    global gemm_dispatch_count
+    gemm_dispatch_count += 1
+    out = _require_ext().linear_add_norm(
+        x.contiguous(), weight, residual.contiguous(),
+        None if norm is None else norm.contiguous(), eps, rounded)
+    return out if norm is not None else (None, out[0])
+
+
+def _freq(inv_freq: torch.Tensor) -> torch.Tensor:
+    # the kernel takes fp32 and bf16 as they are
+    if inv_freq.dtype in (torch.float32, torch.bfloat16):
+        return inv_freq.contiguous()
+    return inv_freq.float()
+
+
+def head_norm_fits(D: int) -> bool:
+    """rope_append_ has the lanes of a head sum their squares among
+    themselves: a power of two of 16 elements each, one wave at most."""
+    return D % 16 == 0 and D <= 1024 and (D & (D - 1)) == 0
+
+
+def linear_rope_append_(x: torch.Tensor, weight: torch.Tensor,
+                        bias: Optional[torch.Tensor], k_cache: torch.Tensor,
+                        v_cache: torch.Tensor, positions: torch.Tensor,
+                        inv_freq: torch.Tensor, S: int, Hq: int, Hkv: int,
+                        block_table: Optional[torch.Tensor] = None,
+                        q_norm: Optional[torch.Tensor] = None,
+                        k_norm: Optional[torch.Tensor] = None,
+                        eps: float = 0.0) -> torch.Tensor:
+    """rope_append_ of x @ weight^T + bias, for a product that
+    serving_gemm() takes: its cuts of K are summed on the way."""
+    global gemm_dispatch_count
+    gemm_dispatch_count += 1
+    return _require_ext().linear_rope_append_(
+        x.contiguous(), weight,
+        bias.to(torch.bfloat16) if bias is not None else None, k_cache,
+        v_cache, positions.int(), _freq(inv_freq), S, Hq, Hkv,
+        block_table.int() if block_table is not None else None,
+        q_norm, k_norm, eps)
+
+
 def rope_append_(qkv: torch.Tensor, k_cache: torch.Tensor,
                  v_cache: torch.Tensor, positions: torch.Tensor,
                  inv_freq: torch.Tensor, S: int, Hq: int, Hkv: int,
-                 block_table: Optional[torch.Tensor] = None) -> torch.Tensor:
+                 block_table: Optional[torch.Tensor] = None,
+                 q_norm: Optional[torch.Tensor] = None,
+                 k_norm: Optional[torch.Tensor] = None,
+                 eps: float = 0.0) -> torch.Tensor:
     """Fused RoPE + KV-cache append from the fused-QKV projection output.
 
     qkv [T, (Hq+2*Hkv)*D] with T = B*S (q | k | v per row); caches
     [B,Hkv,Smax,D] (or paged pools [n_pages,Hkv,128,D] with block_table
     [B, pages]); positions [T] gives the RoPE angle and cache slot.
+    q_norm, k_norm [D] (both or neither): RMSNorm per head of q and k first.
     Returns the rotated q as a contiguous [T, Hq, D] tensor.
     """
+    if q_norm is not None and not (_on_gpu(qkv)
+                                   and head_norm_fits(k_cache.shape[-1])):
+        T, D = qkv.numel() // qkv.shape[-1], k_cache.shape[-1]
+        q, k, v = qkv.split([Hq * D, Hkv * D, Hkv * D], dim=-1)
+        q = rmsnorm(q.reshape(T, Hq, D), q_norm, eps)
+        k = rmsnorm(k.reshape(T, Hkv, D), k_norm, eps)
+        qkv = torch.cat([q.reshape(T, -1), k.reshape(T, -1),
+                         v.reshape(T, -1)], dim=-1)
+        q_norm = k_norm = None
     if _on_gpu(qkv):
         return _require_ext().rope_append_(
             qkv.contiguous(), k_cache, v_cache, positions.int(),
-            inv_freq.float(), S, Hq, Hkv,
-            block_table.int() if block_table is not None else None)
+            _freq(inv_freq), S, Hq, Hkv,
+            block_table.int() if block_table is not None else None,
+            q_norm, k_norm, eps)
     D = k_cache.shape[-1]
     T = qkv.numel() // qkv.shape[-1]
     q = qkv[..., :Hq * D].reshape(T, Hq, D).contiguous()
@@ -282,6 +361,34 @@ def attention_prefill(q, k, v, causal: bool = True,
                                        q_off)
 
 
+def attention_prefill_cache(q, k_cache, v_cache, kv_len: int,
+                            scale: Optional[float] = None,
+                            block_table: Optional[torch.Tensor] = None
+                            ) -> torch.Tensor:
+    """Causal attention of q [B,Sq,Hq,D], the rows at positions
+    kv_len-Sq.., over the first kv_len positions of a cache
+    [B,Hkv,Smax,D] (or paged pools + block_table). Inference path."""
+    S = q.shape[1]
+    if (_on_gpu(q) and q.dtype == torch.bfloat16
+            and q.shape[-1] in (64, 128) and not q.requires_grad):
+        # in place: a copy of K and V in [B,S,H,D] order cost 10 to 25 us a
+        # layer where the attention itself takes 30 to 100
+        return _require_ext().prefill_attn_cache(
+            q.contiguous(), k_cache, v_cache,
+            block_table.int() if block_table is not None else None, kv_len,
+            scale if scale is not None else 1.0 / math.sqrt(q.shape[-1]))
+    if block_table is not None:
+        n = (kv_len + 127) // 128
+        pages = block_table[:, :n].long()
+        k, v = (c[pages].permute(0, 1, 3, 2, 4).flatten(1, 2)[:, :kv_len]
+                for c in (k_cache, v_cache))
+    else:
+        k, v = (c[:, :, :kv_len].permute(0, 2, 1, 3)
+                for c in (k_cache, v_cache))
+    return attention_prefill(q, k.contiguous(), v.contiguous(), causal=True,
+                             scale=scale, q_off=kv_len - S)
+
+
 class _FlashAttnFn(torch.autograd.Function):
     """Hand-written flash attention for training (gfx950): forward =
     prefill kernel saving the logsumexp; backward = the MFMA kernels in
@@ -336,10 +443,11 @@ def attention_train(q, k, v, causal: bool = True,
 
 def attention_decode(q, k_cache, v_cache, seq_lens,
                      scale: Optional[float] = None, n_split: int = 0,
-                     block_table: Optional[torch.Tensor] = None
-                     ) -> torch.Tensor:
+                     block_table: Optional[torch.Tensor] = None,
+                     len_add: int = 0) -> torch.Tensor:
     """q [B,1,Hq,D] or [B,Hq,D]; caches [B,Hkv,Smax,D] (or paged pools +
-    block_table); seq_lens [B]. n_split: flash-decode splits (0 = auto)."""
+    block_table); seq_lens [B], each of them len_add longer. n_split:
+    flash-decode splits (0 = auto)."""
     squeeze = q.dim() == 4
     if squeeze:
         q3 = q.squeeze(1)
@@ -347,6 +455,7 @@ def attention_decode(q, k_cache, v_cache, seq_lens,
         q3 = q
     scale = scale if scale is not None else 1.0 / math.sqrt(q3.shape[-1])
     if not _on_gpu(q3):
+        seq_lens = seq_lens + len_add
         if block_table is not None:
             # gather pages -> contiguous [B, L, Hkv, D] for the reference
             B = q3.shape[0]
@@ -367,7 +476,7 @@ def attention_decode(q, k_cache, v_cache, seq_lens,
         return out if squeeze else out.squeeze(1)
     out = _require_ext().decode_attn(
         q3.contiguous(), k_cache, v_cache, seq_lens.int(), scale, n_split,
-        block_table.int() if block_table is not None else None)
+        block_table.int() if block_table is not None else None, len_add)
     return out.unsqueeze(1) if squeeze else out
 
 
@@ -418,23 +527,26 @@ def _use_tl_gemm(M: int, N: int, K: int) -> bool:
             and _gemm_class(N, K) not in _LIB_CLASSES)
 
 
+def serving_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """x @ weight^T goes to the hand-written family."""
+    return (x.is_cuda and not torch.is_grad_enabled()
+            and x.dtype == torch.bfloat16
+            and not _os.environ.get("TL_NO_SKINNY")
+            and _use_tl_gemm(x.numel() // x.shape[-1], weight.shape[0],
+                             x.shape[-1]))
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor,
            bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x @ W^T + bias. Serving-M shapes route to the hand-written MFMA
     family (skinny_gemm.hip / gemm_tiled.hip); large prefill M and
     training go to torch/hipBLASLt."""
     global gemm_dispatch_count
-    if (x.is_cuda and not torch.is_grad_enabled()
-            and x.dtype == torch.bfloat16
-            and not _os.environ.get("TL_NO_SKINNY")):
-        K = x.shape[-1]
-        M = x.numel() // K
-        N = weight.shape[0]
-        if _use_tl_gemm(M, N, K):
-            gemm_dispatch_count += 1
-            return _require_ext().skinny_gemm(
-                x.contiguous(), weight,
-                bias.to(torch.bfloat16) if bias is not None else None)
+    if serving_gemm(x, weight):
+        gemm_dispatch_count += 1
+        return _require_ext().skinny_gemm(
+            x.contiguous(), weight,
+            bias.to(torch.bfloat16) if bias is not None else None)
     return torch.nn.functional.linear(x, weight, bias)
 
 

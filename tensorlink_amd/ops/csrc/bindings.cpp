@@ -34,11 +34,6 @@ void tl_prefill_attn(const void* q, const void* k, const void* v,
                      int Sq, int Skv, int q_off, int Hq, int Hkv, int D,
                      float scale, int causal, int bt_stride,
                      hipStream_t stream);
-void tl_rope_append(const void* qkv, void* q_out, void* k_cache,
-                    void* v_cache, const void* positions,
-                    const void* inv_freq, const void* block_table,
-                    int64_t T, int row_stride, int S, int Hq, int Hkv,
-                    int D, int Smax, int bt_stride, hipStream_t stream);
 void tl_swiglu_fused(const void* gu, void* out, int64_t N, int I,
                      hipStream_t stream);
 void tl_swiglu_fused_bwd(const void* dout, const void* gu, void* dgu,
@@ -46,12 +41,24 @@ void tl_swiglu_fused_bwd(const void* dout, const void* gu, void* dgu,
 void tl_rope_rows(void* qkv, void* q, void* k, void* v, const void* positions,
                   const void* inv_freq, int64_t T, int Hq, int Hkv, int D,
                   int bwd, hipStream_t stream);
+void tl_add_norm(const void* x, const void* partial, int n_split,
+                 const void* residual, const void* w, void* r_out, void* y,
+                 int64_t M, int H, int rounded, float eps,
+                 hipStream_t stream);
+void tl_rope_append_rows(const void* x, const void* partial, int n_split,
+                         const void* bias, void* q_out, void* k_cache,
+                         void* v_cache, const void* positions,
+                         const void* inv_freq, int freq_bf16,
+                         const void* table, int bt_stride, const void* qw,
+                         const void* kw, float eps, int64_t T, int S, int Hq,
+                         int Hkv, int D, int Smax, hipStream_t stream);
 void tl_decode_attn_mfma(const void* q, const void* k_cache,
                          const void* v_cache, const void* seq_lens,
                          const void* block_table, void* out,
                          void* partial, void* partial_ml, int B, int Hq,
                          int Hkv, int Smax, int D, float scale, int n_split,
-                         int bt_stride, int per_row, hipStream_t stream);
+                         int bt_stride, int per_row, int len_add,
+                         hipStream_t stream);
 void tl_skinny_gemm(const void* x, const void* w, const void* bias,
                     void* out, void* partial, int M, int N, int K,
                     int n_split, int k_per, hipStream_t stream);
@@ -70,11 +77,6 @@ void tl_prefill_attn(const void* q, const void* k, const void* v,
                      int Sq, int Skv, int q_off, int Hq, int Hkv, int D,
                      float scale, int causal, int bt_stride,
                      hipStream_t stream);
-void tl_rope_append(const void* qkv, void* q_out, void* k_cache,
-                    void* v_cache, const void* positions,
-                    const void* inv_freq, const void* block_table,
-                    int64_t T, int row_stride, int S, int Hq, int Hkv,
-                    int D, int Smax, int bt_stride, hipStream_t stream);
 void tl_swiglu_fused(const void* gu, void* out, int64_t N, int I,
                      hipStream_t stream);
 void tl_decode_attn_mfma(const void* q, const void* k_cache,
@@ -82,7 +84,8 @@ void tl_decode_attn_mfma(const void* q, const void* k_cache,
                          const void* block_table, void* out,
                          void* partial, void* partial_ml, int B, int Hq,
                          int Hkv, int Smax, int D, float scale, int n_split,
-                         int bt_stride, int per_row, hipStream_t stream);
+                         int bt_stride, int per_row, int len_add,
+                         hipStream_t stream);
 void tl_skinny_gemm(const void* x, const void* w, const void* bias,
                     void* out, void* partial, int M, int N, int K,
                     int n_split, int k_per, hipStream_t stream);
@@ -224,7 +227,7 @@ void adamw_(Tensor param, Tensor grad, Tensor m, Tensor v, double lr,
 
 Tensor decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor seq_lens,
                    double scale, int64_t n_split,
-                   c10::optional<Tensor> block_table) {
+                   c10::optional<Tensor> block_table, int64_t len_add) {
   CHECK_IN(q, torch::kBFloat16);
   CHECK_IN(k_cache, torch::kBFloat16);
   CHECK_IN(v_cache, torch::kBFloat16);
@@ -247,6 +250,7 @@ Tensor decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor seq_lens,
   const bool legacy = (getenv("TL_DECODE_LEGACY") != nullptr || G > 16) &&
                       bt == nullptr;
   if (legacy) {
+    if (len_add) seq_lens = seq_lens + len_add;
     tl_decode_attn(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                    seq_lens.data_ptr(), out.data_ptr(), B, Hq, Hkv, Smax, D,
                    (float)scale, cur_stream());
@@ -276,7 +280,7 @@ Tensor decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor seq_lens,
   tl_decode_attn_mfma(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                       seq_lens.data_ptr(), bt, out.data_ptr(), pp, pml, B,
                       Hq, Hkv, Smax, D, (float)scale, (int)n_split,
-                      bt_stride, per_row, cur_stream());
+                      bt_stride, per_row, (int)len_add, cur_stream());
   return out;
 }
 
@@ -334,6 +338,37 @@ std::vector<Tensor> prefill_attn_lse(Tensor q, Tensor k, Tensor v,
   return {out, lse};
 }
 
+// Causal attention of q's rows (positions kv_len - Sq ..) over the first
+// kv_len positions of a cache, read in place: [B,Hkv,Smax,D] or page pools.
+Tensor prefill_attn_cache(Tensor q, Tensor k_cache, Tensor v_cache,
+                          c10::optional<Tensor> table, int64_t kv_len,
+                          double scale) {
+  CHECK_IN(q, torch::kBFloat16);
+  CHECK_IN(k_cache, torch::kBFloat16);
+  CHECK_IN(v_cache, torch::kBFloat16);
+  const int64_t Sq = q.size(1), D = q.size(3);
+  const int64_t Hkv = k_cache.size(1), Smax = k_cache.size(2);
+  TORCH_CHECK(k_cache.size(3) == D && v_cache.sizes() == k_cache.sizes(),
+              "cache shape mismatch");
+  TORCH_CHECK(Sq > 0 && Sq <= kv_len, "kv_len must cover the query rows");
+  const int* bt = nullptr;
+  int bt_stride = 0;
+  if (table.has_value()) {
+    CHECK_IN(table.value(), torch::kInt);
+    TORCH_CHECK(Smax == 128, "paged pool PAGE must be 128");
+    TORCH_CHECK(table->size(0) == q.size(0) && table->size(1) * 128 >= kv_len,
+                "table too small");
+    bt = table->data_ptr<int>();
+    bt_stride = (int)table->size(1);
+  } else {
+    TORCH_CHECK(k_cache.size(0) == q.size(0) && kv_len <= Smax,
+                "cache too small");
+  }
+  return prefill_run(q, k_cache, v_cache, bt, bt_stride, Hkv * Smax * D,
+                     Smax * D, D, kv_len, Hkv, scale, true, kv_len - Sq,
+                     nullptr);
+}
+
 std::vector<Tensor> attn_bwd(Tensor q, Tensor k, Tensor v, Tensor dout,
                              Tensor out, Tensor lse, double scale,
                              bool causal) {
@@ -367,44 +402,6 @@ std::vector<Tensor> attn_bwd(Tensor q, Tensor k, Tensor v, Tensor dout,
               parts > 1 ? sums[1].data_ptr() : nullptr, B, S, Hq, Hkv, D,
               (float)scale, causal ? 1 : 0, parts, cur_stream());
   return {dq, dk, dv};
-}
-
-// qkv: [T, row_stride] fused projection output (q | k | v per row).
-// Returns rotated q as a contiguous [T, Hq, D] tensor; k/v land in the
-// caches.
-Tensor rope_append_(Tensor qkv, Tensor k_cache, Tensor v_cache,
-                    Tensor positions, Tensor inv_freq, int64_t S,
-                    int64_t Hq, int64_t Hkv,
-                    c10::optional<Tensor> block_table) {
-  CHECK_IN(qkv, torch::kBFloat16);
-  CHECK_IN(k_cache, torch::kBFloat16);
-  CHECK_IN(v_cache, torch::kBFloat16);
-  CHECK_IN(positions, torch::kInt);
-  CHECK_IN(inv_freq, torch::kFloat);
-  const int D = k_cache.size(3);
-  const int row_stride = qkv.size(-1);
-  TORCH_CHECK(row_stride == (Hq + 2 * Hkv) * D, "qkv width mismatch");
-  const int64_t T = qkv.numel() / row_stride;
-  const int Smax = k_cache.size(2);
-  TORCH_CHECK(T % S == 0, "T must be divisible by S");
-  TORCH_CHECK(D % 16 == 0, "D must be divisible by 16");
-  const void* bt = nullptr;
-  int bt_stride = 0;
-  if (block_table.has_value()) {
-    CHECK_IN(block_table.value(), torch::kInt);
-    TORCH_CHECK(k_cache.size(2) == 128, "paged pool PAGE must be 128");
-    bt = block_table->data_ptr();
-    bt_stride = block_table->size(1);
-    TORCH_CHECK(block_table->size(0) * S == T, "table batch mismatch");
-  } else {
-    TORCH_CHECK(k_cache.size(0) * S == T, "cache batch mismatch");
-  }
-  auto q_out = torch::empty({T, Hq, (int64_t)D}, qkv.options());
-  tl_rope_append(qkv.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(),
-                 v_cache.data_ptr(), positions.data_ptr(),
-                 inv_freq.data_ptr(), bt, T, row_stride, (int)S, (int)Hq,
-                 (int)Hkv, D, Smax, bt_stride, cur_stream());
-  return q_out;
 }
 
 Tensor swiglu_fused(Tensor gu) {
@@ -505,7 +502,19 @@ static GemmSplit gemm_split(int N, int K) {
   return {(steps + per - 1) / per, per * 256};
 }
 
-Tensor skinny_gemm(Tensor x, Tensor w, c10::optional<Tensor> bias) {
+// x W^T of the family: bf16 rows in `out`, or its cuts in `partial` where the
+// caller sums them (cuts set) and there are any.
+struct Product {
+  Tensor out, partial;
+  int n_split = 1;
+  const void* rows() const { return out.defined() ? out.data_ptr() : nullptr; }
+  const void* cuts() const {
+    return partial.defined() ? partial.data_ptr() : nullptr;
+  }
+};
+
+Product run_gemm(const Tensor& x, const Tensor& w,
+                 const c10::optional<Tensor>& bias, bool cuts) {
   CHECK_IN(x, torch::kBFloat16);
   CHECK_IN(w, torch::kBFloat16);
   const int K = x.size(-1);
@@ -513,29 +522,170 @@ Tensor skinny_gemm(Tensor x, Tensor w, c10::optional<Tensor> bias) {
   const int N = w.size(0);
   TORCH_CHECK(w.size(1) == K, "K mismatch");
   TORCH_CHECK(K % 32 == 0 && N % 64 == 0, "unsupported shape");
-  auto sizes = x.sizes().vec();
-  sizes.back() = N;
-  auto out = torch::empty(sizes, x.options());
   const void* bp = nullptr;
   if (bias.has_value()) {
     CHECK_IN(bias.value(), torch::kBFloat16);
     bp = bias->data_ptr();
   }
   const auto [n_split, k_per] = gemm_split(N, K);
-  Tensor partial;
-  void* pp = nullptr;
-  if (n_split > 1) {
-    partial = torch::empty({(int64_t)n_split * M * N},
-                           x.options().dtype(torch::kFloat));
-    pp = partial.data_ptr();
+  Product p;
+  p.n_split = n_split;
+  if (n_split > 1)
+    p.partial = torch::empty({(int64_t)n_split * M * N},
+                             x.options().dtype(torch::kFloat));
+  if (!cuts || n_split == 1) {
+    auto sizes = x.sizes().vec();
+    sizes.back() = N;
+    p.out = torch::empty(sizes, x.options());
   }
+  void* op = p.out.defined() ? p.out.data_ptr() : nullptr;
+  void* pp = n_split > 1 ? p.partial.data_ptr() : nullptr;
   if (M <= 64)
-    tl_skinny_gemm(x.data_ptr(), w.data_ptr(), bp, out.data_ptr(), pp,
-                   (int)M, N, K, n_split, k_per, cur_stream());
+    tl_skinny_gemm(x.data_ptr(), w.data_ptr(), bp, op, pp, (int)M, N, K,
+                   n_split, k_per, cur_stream());
   else
-    tl_gemm_tiled(x.data_ptr(), w.data_ptr(), bp, out.data_ptr(), pp,
-                  (int)M, N, K, n_split, k_per, cur_stream());
-  return out;
+    tl_gemm_tiled(x.data_ptr(), w.data_ptr(), bp, op, pp, (int)M, N, K,
+                  n_split, k_per, cur_stream());
+  return p;
+}
+
+Tensor skinny_gemm(Tensor x, Tensor w, c10::optional<Tensor> bias) {
+  return run_gemm(x, w, bias, false).out;
+}
+
+// r = x (+ residual), y = RMSNorm(r) w; y undefined without w
+std::vector<Tensor> add_norm_run(const Product& p, const Tensor& residual,
+                                 const c10::optional<Tensor>& w, double eps,
+                                 bool rounded) {
+  CHECK_IN(residual, torch::kBFloat16);
+  const int64_t H = residual.size(-1), M = residual.numel() / H;
+  TORCH_CHECK(H % 8 == 0 && H <= 16384, "width must be a multiple of 8");
+  auto r = torch::empty_like(residual);
+  Tensor y;
+  if (w.has_value()) {
+    CHECK_IN(w.value(), torch::kBFloat16);
+    TORCH_CHECK(w->numel() == H, "norm weight size mismatch");
+    y = torch::empty_like(residual);
+  }
+  tl_add_norm(p.rows(), p.cuts(), p.n_split, residual.data_ptr(),
+              w.has_value() ? w->data_ptr() : nullptr, r.data_ptr(),
+              w.has_value() ? y.data_ptr() : nullptr, M, (int)H,
+              rounded ? 1 : 0, (float)eps, cur_stream());
+  if (w.has_value()) return {y, r};
+  return {r};
+}
+
+std::vector<Tensor> add_norm(Tensor x, Tensor residual,
+                             c10::optional<Tensor> w, double eps,
+                             bool rounded) {
+  CHECK_IN(x, torch::kBFloat16);
+  TORCH_CHECK(x.sizes() == residual.sizes(), "shapes differ");
+  Product p;
+  p.out = x;
+  return add_norm_run(p, residual, w, eps, rounded);
+}
+
+std::vector<Tensor> linear_add_norm(Tensor x, Tensor weight, Tensor residual,
+                                    c10::optional<Tensor> w, double eps,
+                                    bool rounded) {
+  TORCH_CHECK(residual.size(-1) == weight.size(0) &&
+                  residual.numel() / residual.size(-1) ==
+                      x.numel() / x.size(-1),
+              "residual shape mismatch");
+  Product p = run_gemm(x, weight, c10::nullopt, true);
+  if (p.out.defined()) p.partial = Tensor();
+  return add_norm_run(p, residual, w, eps, rounded);
+}
+
+Tensor rope_append_run(const Product& p, const Tensor& like,
+                       const c10::optional<Tensor>& bias, Tensor& k_cache,
+                       Tensor& v_cache, const Tensor& positions,
+                       const Tensor& inv_freq, int64_t S, int64_t Hq,
+                       int64_t Hkv, const c10::optional<Tensor>& table,
+                       const c10::optional<Tensor>& qw,
+                       const c10::optional<Tensor>& kw, double eps,
+                       int64_t T) {
+  CHECK_IN(k_cache, torch::kBFloat16);
+  CHECK_IN(v_cache, torch::kBFloat16);
+  CHECK_IN(positions, torch::kInt);
+  TORCH_CHECK(inv_freq.is_cuda() && inv_freq.is_contiguous() &&
+                  (inv_freq.scalar_type() == torch::kFloat ||
+                   inv_freq.scalar_type() == torch::kBFloat16),
+              "inv_freq must be fp32 or bf16 on GPU");
+  const int64_t D = k_cache.size(3), Smax = k_cache.size(2);
+  TORCH_CHECK(v_cache.sizes() == k_cache.sizes() && k_cache.size(1) == Hkv,
+              "cache shapes mismatch");
+  TORCH_CHECK(D % 16 == 0, "D must be divisible by 16");
+  TORCH_CHECK(inv_freq.numel() * 2 == D && positions.numel() == T,
+              "positions or inv_freq size mismatch");
+  TORCH_CHECK(T % S == 0, "T must be divisible by S");
+  const int* bt = nullptr;
+  int bt_stride = 0;
+  if (table.has_value()) {
+    CHECK_IN(table.value(), torch::kInt);
+    TORCH_CHECK(Smax == 128, "paged pool PAGE must be 128");
+    TORCH_CHECK(table->size(0) * S == T, "table batch mismatch");
+    bt = table->data_ptr<int>();
+    bt_stride = (int)table->size(1);
+  } else {
+    TORCH_CHECK(k_cache.size(0) * S == T, "cache batch mismatch");
+  }
+  const void *qp = nullptr, *kp = nullptr;
+  if (qw.has_value()) {
+    CHECK_IN(qw.value(), torch::kBFloat16);
+    TORCH_CHECK(kw.has_value(), "q and k norms go together");
+    CHECK_IN(kw.value(), torch::kBFloat16);
+    TORCH_CHECK(qw->numel() == D && kw->numel() == D &&
+                    D <= 1024 && ((D / 16) & (D / 16 - 1)) == 0,
+                "norms need D / 16 to be a power of two up to 64");
+    qp = qw->data_ptr();
+    kp = kw->data_ptr();
+  }
+  auto q = torch::empty({T, Hq, D}, like.options());
+  tl_rope_append_rows(p.rows(), p.cuts(), p.n_split,
+                      bias.has_value() ? bias->data_ptr() : nullptr,
+                      q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                      positions.data_ptr(), inv_freq.data_ptr(),
+                      inv_freq.scalar_type() == torch::kBFloat16 ? 1 : 0, bt,
+                      bt_stride, qp, kp, (float)eps, T, (int)S, (int)Hq,
+                      (int)Hkv, (int)D, (int)Smax, cur_stream());
+  return q;
+}
+
+// qkv: [T, (Hq + 2 Hkv) D] fused projection output (q | k | v per row).
+// Returns (normed and) rotated q [T, Hq, D]; k and v land in the caches.
+Tensor rope_append_(Tensor qkv, Tensor k_cache, Tensor v_cache,
+                    Tensor positions, Tensor inv_freq, int64_t S, int64_t Hq,
+                    int64_t Hkv, c10::optional<Tensor> block_table,
+                    c10::optional<Tensor> qw, c10::optional<Tensor> kw,
+                    double eps) {
+  CHECK_IN(qkv, torch::kBFloat16);
+  TORCH_CHECK(qkv.size(-1) == (Hq + 2 * Hkv) * k_cache.size(3),
+              "qkv width mismatch");
+  Product p;
+  p.out = qkv;
+  return rope_append_run(p, qkv, c10::nullopt, k_cache, v_cache, positions,
+                         inv_freq, S, Hq, Hkv, block_table, qw, kw, eps,
+                         qkv.numel() / qkv.size(-1));
+}
+
+// The fused projection itself in front of it.
+Tensor linear_rope_append_(Tensor x, Tensor weight,
+                           c10::optional<Tensor> bias, Tensor k_cache,
+                           Tensor v_cache, Tensor positions, Tensor inv_freq,
+                           int64_t S, int64_t Hq, int64_t Hkv,
+                           c10::optional<Tensor> block_table,
+                           c10::optional<Tensor> qw,
+                           c10::optional<Tensor> kw, double eps) {
+  TORCH_CHECK(weight.size(0) == (Hq + 2 * Hkv) * k_cache.size(3) &&
+                  (!bias.has_value() || bias->numel() == weight.size(0)),
+              "qkv width mismatch");
+  Product p = run_gemm(x, weight, bias, true);
+  const bool done = p.out.defined();         // bias is in there
+  if (done) p.partial = Tensor();
+  return rope_append_run(p, x, done ? c10::nullopt : bias, k_cache, v_cache,
+                         positions, inv_freq, S, Hq, Hkv, block_table, qw, kw,
+                         eps, x.numel() / x.size(-1));
 }
 
 Tensor sample_tokens(Tensor logits, Tensor temps, Tensor top_ps,
@@ -595,7 +745,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
   register_gla_ops(mod);
   register_delta_ops(mod);
   mod.def("rope_append_", &rope_append_,
-          "fused RoPE + KV-cache append from fused-QKV rows");
+          "(norm +) RoPE rotate + KV-cache append from fused-QKV rows",
+          py::arg("qkv"), py::arg("k_cache"), py::arg("v_cache"),
+          py::arg("positions"), py::arg("inv_freq"), py::arg("S"),
+          py::arg("Hq"), py::arg("Hkv"), py::arg("block_table"),
+          py::arg("qw") = py::none(), py::arg("kw") = py::none(),
+          py::arg("eps") = 0.0);
+  mod.def("linear_rope_append_", &linear_rope_append_,
+          "fused-QKV projection with rope_append_ on its cuts");
+  mod.def("add_norm", &add_norm, "residual add (+ RMSNorm)");
+  mod.def("linear_add_norm", &linear_add_norm,
+          "projection, residual add (+ RMSNorm)");
   mod.def("swiglu_fused", &swiglu_fused, "silu-mul on fused [.,2I] rows");
   mod.def("skinny_gemm", &skinny_gemm, "decode-M GEMM: x @ W^T + bias");
   mod.def("rmsnorm_fwd", &rmsnorm_fwd, "fused RMSNorm fwd (+residual)");
@@ -610,8 +770,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
           "fused projection rows to rotated q, k, and v");
   mod.def("rope_merge", &rope_merge,
           "gradients of q, k, v rotated back into projection rows");
-  mod.def("decode_attn", &decode_attn, "GQA decode attention over KV cache");
+  mod.def("decode_attn", &decode_attn, "GQA decode attention over KV cache",
+          py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
+          py::arg("seq_lens"), py::arg("scale"), py::arg("n_split"),
+          py::arg("block_table"), py::arg("len_add") = 0);
   mod.def("prefill_attn", &prefill_attn, "causal GQA prefill attention");
+  mod.def("prefill_attn_cache", &prefill_attn_cache,
+          "the same with K and V read from a cache in place");
   mod.def("sample_tokens", &sample_tokens,
           "fused penalties/temperature/top-k/top-p sampling, one block/row");
   mod.def("bump_sample_counter", &bump_sample_counter,

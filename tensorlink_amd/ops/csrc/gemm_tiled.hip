@@ -288,7 +288,8 @@ extern "C" {
 void tl_gemm_reduce(const void* partial, const void* bias, void* out,
                     int64_t MN, int N, int n_split, hipStream_t stream);
 
-// partial: scratch [n_split * M * N] floats (only used when n_split > 1).
+// partial: scratch [n_split * M * N] floats (only used when n_split > 1; out
+// null then: the cuts are left for the caller to sum).
 //
 // The tile is the one that needs no second round of blocks: BN 64 with four
 // buffers (one block per CU) while that makes at most 256 blocks, else BN 128
@@ -328,7 +329,7 @@ void tl_gemm_tiled(const void* x, const void* w, const void* bias, void* out,
     if (n_split > 1) TL_GT(128, 2, 1, b128); else TL_GT(128, 2, 0, b128);
   }
 #undef TL_GT
-  if (n_split > 1)
+  if (n_split > 1 && out)
     tl_gemm_reduce(partial, bias, out, (int64_t)M * N, N, n_split, stream);
 }
 

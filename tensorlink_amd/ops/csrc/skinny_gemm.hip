@@ -174,7 +174,8 @@ void tl_gemm_reduce(const void* partial, const void* bias, void* out,
                      (const bf16*)bias, (bf16*)out, MN, N, n_split);
 }
 
-// partial: scratch [n_split * M * N] floats (only used when n_split > 1)
+// partial: scratch [n_split * M * N] floats (only used when n_split > 1; out
+// null then: the cuts are left for the caller to sum)
 void tl_skinny_gemm(const void* x, const void* w, const void* bias,
                     void* out, void* partial, int M, int N, int K,
                     int n_split, int k_per, hipStream_t stream) {
@@ -195,7 +196,7 @@ void tl_skinny_gemm(const void* x, const void* w, const void* bias,
   else if (M <= 32) TL_SG(2);
   else TL_SG(4);
 #undef TL_SG
-  if (n_split > 1)
+  if (n_split > 1 && out)
     tl_gemm_reduce(partial, bias, out, (int64_t)M * N, N, n_split, stream);
 }
 

@@ -911,3 +911,122 @@ def test_training_step_uses_flash_bwd():
     losses = [t.train_step(ids, labels=ids) for _ in range(4)]
     assert all(torch.isfinite(torch.tensor(losses)))
     assert losses[-1] < losses[0], losses
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("H,K,M", [
+    (64, 32, 1), (2048, 96, 3), (2112, 2080, 65),      # one cut, four
+    (8192, 800, 33), (16384, 288, 2)])
+def test_linear_add_norm(H, K, M):
+    """The cuts of a product summed by the norm behind it: the rows that the
+    product alone writes, and their sum with the residual, to the bit; the
+    norm against fp64 (its result is rounded to bf16, 2^-9)."""
+    ops = _ext()
+    torch.manual_seed(H + K)
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    x, w, res, g = mk(M, K), mk(H, K) / K ** 0.5, mk(M, H), mk(H)
+    rows = ops._require_ext().skinny_gemm(x, w, None)
+    r = rows + res
+    none, alone = ops.linear_add_norm(x, w, res, None, 1e-6, True)
+    assert none is None and torch.equal(alone, r)
+    for rounded in (True, False):
+        f = r.double() if rounded else rows.double() + res.double()
+        want = f * (f.pow(2).mean(-1, keepdim=True) + 1e-6).rsqrt() * g.double()
+        got = [ops.linear_add_norm(x, w, res, g, 1e-6, rounded)]
+        if rounded:
+            got.append(ops.add_norm(rows, res, g, 1e-6))
+        for y, rr in got:
+            assert torch.equal(rr, r)
+            assert (y.double() - want).norm() / want.norm() < 3e-3
+            assert torch.equal(y, got[0][0])
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("Hq,Hkv,D,S", [
+    (2, 2, 16, 3), (3, 1, 48, 1), (28, 4, 128, 5), (5, 5, 2048, 2)])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("freq", [torch.float32, torch.bfloat16])
+def test_rope_append_rows(Hq, Hkv, D, S, norm, freq):
+    """Norm, rotation and append of a product's rows against fp64 (two
+    roundings to bf16 and sine and cosine of 2^-20 at most: 2-norm error under
+    6e-3); values are bits. From the rows or from the product's cuts, on a
+    contiguous or a paged cache: the same bits. Nothing else is written."""
+    ops = _ext()
+    torch.manual_seed(D)
+    B, K, Smax = 2, 544, 384
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    N = (Hq + 2 * Hkv) * D
+    N64 = -(-N // 64) * 64 == N
+    x, w, b = mk(B * S, K), mk(N, K) / K ** 0.5, mk(N)
+    rows = (ops._require_ext().skinny_gemm(x, w, b) if N64
+            else torch.nn.functional.linear(x, w, b))
+    inv = (1e4 ** -(torch.arange(0, D, 2, device=DEV) / D)).to(freq)
+    start = torch.tensor([0, 129], device=DEV, dtype=torch.int32)
+    pos = (start[:, None] + torch.arange(S, device=DEV,
+                                         dtype=torch.int32)).reshape(-1)
+    qw, kw = (mk(D), mk(D)) if norm else (None, None)
+    q, k, v = (t.reshape(B * S, -1, D) for t in rows.double().split(
+        [Hq * D, Hkv * D, Hkv * D], 1))
+    if norm:
+        q, k = (t * (t.pow(2).mean(-1, keepdim=True) + 1e-6).rsqrt()
+                * g.double() for t, g in ((q, qw), (k, kw)))
+    ang = pos.double()[:, None, None] * inv.double()
+    c, s = ang.cos(), ang.sin()
+    turn = lambda t: torch.cat([t[..., :D // 2] * c - t[..., D // 2:] * s,
+                                t[..., D // 2:] * c + t[..., :D // 2] * s], -1)
+    q, k = turn(q), turn(k)
+    table = torch.randperm(B * 3, device=DEV).int().view(B, 3)
+    first = None
+    for paged in (False, True):
+        for cuts in (False, True) if N64 and (
+                not norm or ops.head_norm_fits(D)) else (False,):
+            shape = (B * 3, Hkv, 128, D) if paged else (B, Hkv, Smax, D)
+            kc = torch.full(shape, 7.0, device=DEV, dtype=torch.bfloat16)
+            vc = kc.clone()
+            args = (kc, vc, pos, inv, S, Hq, Hkv, table if paged else None,
+                    qw, kw, 1e-6)
+            out = (ops.linear_rope_append_(x, w, b, *args) if cuts
+                   else ops.rope_append_(rows, *args))
+            if paged:
+                kc, vc = (t[table.long()].transpose(1, 2).reshape(
+                    B, Hkv, Smax, D) for t in (kc, vc))
+            i = pos.long().view(B, 1, S, 1).expand(B, Hkv, S, D)
+            at = lambda t: t.gather(2, i).transpose(1, 2).reshape(
+                B * S, Hkv, D)
+            assert (out.double() - q).norm() / q.norm() < 6e-3
+            assert (at(kc).double() - k).norm() / k.norm() < 6e-3
+            assert torch.equal(at(vc).double(), v)
+            seen = torch.ones_like(kc, dtype=torch.bool).scatter_(2, i, False)
+            assert (kc[seen] == 7).all() and (vc[seen] == 7).all()
+            first = first or (out, kc, vc)
+            assert all(torch.equal(t, f)
+                       for t, f in zip((out, kc, vc), first))
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("S,off,D", [
+    (2, 0, 64), (65, 0, 128), (40, 88, 128), (513, 130, 64), (30, 1100, 128)])
+def test_prefill_attn_reads_cache_in_place(S, off, D):
+    """The bits of attention over the copied keys and values; what lies past
+    the last key is NaN and not seen."""
+    ops = _ext()
+    torch.manual_seed(S)
+    B, Hq, Hkv, n = 2, 6, 2, off + S
+    pages = (n + 127) // 128 + 1
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    q = mk(B, S, Hq, D)
+    k, v = mk(B, Hkv, pages * 128, D), mk(B, Hkv, pages * 128, D)
+    k[:, :, n:], v[:, :, n:] = math.nan, math.nan
+    want = ops.attention_prefill(q, *(t[:, :, :n].transpose(1, 2).contiguous()
+                                      for t in (k, v)), q_off=off)
+    assert torch.equal(ops.attention_prefill_cache(q, k, v, n), want)
+    table = torch.randperm(B * pages, device=DEV).int().view(B, pages)
+    pools = []
+    for t in (k, v):
+        p = torch.empty(B * pages, Hkv, 128, D, device=DEV,
+                        dtype=torch.bfloat16)
+        p[table.long().view(-1)] = t.view(B, Hkv, pages, 128, D).transpose(
+            1, 2).reshape(-1, Hkv, 128, D)
+        pools.append(p)
+    assert torch.equal(ops.attention_prefill_cache(q, *pools, n,
+                                                   block_table=table), want)
