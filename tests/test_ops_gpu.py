@@ -1030,3 +1030,19 @@ def test_prefill_attn_reads_cache_in_place(S, off, D):
         pools.append(p)
     assert torch.equal(ops.attention_prefill_cache(q, *pools, n,
                                                    block_table=table), want)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("N,K", [(9000 // 64 * 64, 544), (65600, 96)])
+def test_tl_gemm_large_tiles(N, K):
+    """The tiles of 256 rows or columns at their edges, with the bits of the
+    few-row kernels (which have their own test against fp64)."""
+    C = _ext()._require_ext()
+    torch.manual_seed(N)
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) / K ** 0.5
+    b = torch.randn(N, device=DEV, dtype=torch.bfloat16)
+    x = torch.randn(513, K, device=DEV, dtype=torch.bfloat16)
+    few = torch.cat([C.skinny_gemm(t.contiguous(), w, b)
+                     for t in x.split(48)])
+    for M in (128, 129, 256, 257, 384, 385, 512, 513):
+        assert torch.equal(C.skinny_gemm(x[:M].contiguous(), w, b), few[:M])
