@@ -78,11 +78,15 @@ def _unwatched(module: nn.Module) -> bool:
                 or nn.modules.module._has_any_global_hook())
 
 
+def _bare(linear: nn.Module) -> bool:
+    """linear(x) is a product and nothing else."""
+    return type(linear) is TLLinear and _unwatched(linear)
+
+
 def _serving(linear: nn.Module, x: torch.Tensor) -> bool:
-    """linear(x) is one product of the serving GEMM family and nothing else,
-    so that what follows may take its fp32 cuts of K as they are."""
-    return (type(linear) is TLLinear and _unwatched(linear)
-            and ops.serving_gemm(x, linear.weight))
+    """linear(x) is one product of the serving GEMM family, so that what
+    follows may take its fp32 cuts of K as they are."""
+    return _bare(linear) and ops.serving_gemm(x, linear.weight)
 
 
 def cached_rows(kv_cache) -> int:
@@ -247,7 +251,11 @@ class MLP(nn.Module):
 
     def inner(self, x):
         """All of it but the down projection."""
-        gu = self.gate_up_proj(x)
+        proj = self.gate_up_proj
+        if (_bare(proj) and proj.bias is None
+                and ops.serving_glu(x, proj.weight)):
+            return ops.linear_swiglu(x, proj.weight)
+        gu = proj(x)
         if (torch.is_grad_enabled() and gu.requires_grad
                 and (not gu.is_cuda or self.inter % 8)):
             gate, up = gu.split([self.inter, self.inter], dim=-1)

@@ -503,10 +503,11 @@ gemm_dispatch_count = 0
 # (N,K)-pure shape classes; TL_GEMM_LIB_CLASSES routes whole classes to
 # hipBLASLt for in-pipeline A/B (a class flips for ALL M at once, so the
 # bitwise M-independence guarantee is preserved per process)
-# default: the gateup class (16k <= N < 64k) routes to hipBLASLt — the
-# BN=64/256 custom structures both lose ~40 us there in-pipeline
-# (profiles/gemm_family_ab.md); all other classes are custom, keeping
-# bitwise M-independence by construction where the tests assert it
+# default: the gateup class (16k <= N < 64k) routes to hipBLASLt, which is
+# faster there above 64 rows (37888 x 3584, 128 / 333 / 512 rows: 67 / 113 /
+# 137 us against 82 / 133 / 176) — all but its few rows with the activation,
+# serving_glu(); all other classes are custom, keeping bitwise M-independence
+# by construction where the tests assert it
 _LIB_CLASSES = frozenset(
     c for c in _os.environ.get("TL_GEMM_LIB_CLASSES",
                                "gateup").split(",") if c)
@@ -534,6 +535,28 @@ def serving_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and not _os.environ.get("TL_NO_SKINNY")
             and _use_tl_gemm(x.numel() // x.shape[-1], weight.shape[0],
                              x.shape[-1]))
+
+
+def serving_glu(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """swiglu(x @ weight^T) of a fused gate and up projection goes to one
+    launch: the streaming kernel, uncut, whose lanes end with both halves.
+    The lines (rows, blocks) are where it stops to be faster than the
+    library's product and the activation behind it (skinny_gemm.hip)."""
+    K = x.shape[-1]
+    M, N = x.numel() // K, weight.shape[0]
+    return (x.is_cuda and not torch.is_grad_enabled()
+            and x.dtype == torch.bfloat16
+            and not _os.environ.get("TL_NO_SKINNY") and M > 0
+            and K % 32 == 0 and N % 64 == 0
+            and _gemm_class(N, K) == "gateup"
+            and M <= (32 if N > 32768 else 64))
+
+
+def linear_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """swiglu of x @ weight^T where serving_glu() takes it."""
+    global gemm_dispatch_count
+    gemm_dispatch_count += 1
+    return _require_ext().skinny_glu(x.contiguous(), weight)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor,

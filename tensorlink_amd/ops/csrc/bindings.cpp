@@ -41,6 +41,8 @@ void tl_swiglu_fused_bwd(const void* dout, const void* gu, void* dgu,
 void tl_rope_rows(void* qkv, void* q, void* k, void* v, const void* positions,
                   const void* inv_freq, int64_t T, int Hq, int Hkv, int D,
                   int bwd, hipStream_t stream);
+void tl_skinny_glu(const void* x, const void* w, void* out, int M, int N,
+                   int K, hipStream_t stream);
 void tl_add_norm(const void* x, const void* partial, int n_split,
                  const void* residual, const void* w, void* r_out, void* y,
                  int64_t M, int H, int rounded, float eps,
@@ -553,6 +555,22 @@ Tensor skinny_gemm(Tensor x, Tensor w, c10::optional<Tensor> bias) {
   return run_gemm(x, w, bias, false).out;
 }
 
+// silu(x gate^T) (x up^T) with w = [gate; up], at most 64 rows
+Tensor skinny_glu(Tensor x, Tensor w) {
+  CHECK_IN(x, torch::kBFloat16);
+  CHECK_IN(w, torch::kBFloat16);
+  const int64_t K = x.size(-1), M = x.numel() / K, N = w.size(0);
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == K, "K mismatch");
+  TORCH_CHECK(M <= 64 && K % 32 == 0 && N % 64 == 0, "unsupported shape");
+  auto sizes = x.sizes().vec();
+  sizes.back() = N / 2;
+  auto out = torch::empty(sizes, x.options());
+  if (M > 0)
+    tl_skinny_glu(x.data_ptr(), w.data_ptr(), out.data_ptr(), (int)M, (int)N,
+                  (int)K, cur_stream());
+  return out;
+}
+
 // r = x (+ residual), y = RMSNorm(r) w; y undefined without w
 std::vector<Tensor> add_norm_run(const Product& p, const Tensor& residual,
                                  const c10::optional<Tensor>& w, double eps,
@@ -757,6 +775,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
   mod.def("linear_add_norm", &linear_add_norm,
           "projection, residual add (+ RMSNorm)");
   mod.def("swiglu_fused", &swiglu_fused, "silu-mul on fused [.,2I] rows");
+  mod.def("skinny_glu", &skinny_glu,
+          "decode-M SwiGLU of a fused gate and up projection");
   mod.def("skinny_gemm", &skinny_gemm, "decode-M GEMM: x @ W^T + bias");
   mod.def("rmsnorm_fwd", &rmsnorm_fwd, "fused RMSNorm fwd (+residual)");
   mod.def("rmsnorm_bwd", &rmsnorm_bwd, "RMSNorm bwd");

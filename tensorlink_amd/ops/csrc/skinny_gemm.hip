@@ -6,8 +6,8 @@
 // how many bytes of W are in flight and how few launches surround it.
 //
 // A block covers 64 rows of W and all rows of x. Both go to LDS by
-// global_load_lds (256 contiguous bytes per row, 16-byte slots permuted by
-// row, so the ds_read_b128 meet no conflicts), three steps of 128 k ahead in
+// global_load_lds (128 or 256 contiguous bytes per row, 16-byte slots permuted by
+// row, so the ds_read_b128 meet no conflicts), three steps of XK k ahead in
 // four buffers. The copies are counted: a step waits for the oldest only, with
 // one barrier. W through registers instead is 64 bytes per row and load, and
 // the compiler then drains all copies at each use. A wave owns 16 rows of W
@@ -19,7 +19,7 @@
 // registers, one step ahead, a barrier that drained it): 3584 x 18944 44 / 45
 // / 53 -> 28 / 28 / 35 us (4.9 TB/s), 4096 x 12288 46 / 47 / 53 -> 21 / 22 /
 // 25, 4608 x 3584 19 / 19 / 22 -> 11 / 11 / 15, 152064 x 3584 241 / 253 / 291
-// -> 179 / 186 / 232 (6.1 TB/s). Cuts inside the block, each with a wave's own
+// -> 179 / 186 / 225 (6.1 TB/s). Cuts inside the block, each with a wave's own
 // buffers and no partials, were slower (44 us on 3584 x 18944).
 //
 // Contract with gemm_tiled.hip: every row sums K in 32-wide
@@ -40,10 +40,12 @@ DEVINLINE void waitcnt_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-constexpr int XK = 128;              // k per step
 constexpr int NB = 4;                // buffers
 
-template <int MT, int SPLIT>
+// XK k per step. GLU: W is [gate; up] of N / 2 rows each and a wave owns eight
+// rows of either at the same columns; out [M, N / 2] = silu(gate) up, of the
+// two rounded to bf16 as the product alone would be.
+template <int MT, int XK, int SPLIT, int GLU>
 __global__ __launch_bounds__(BLOCK) void skinny_gemm_kernel(
     const bf16* __restrict__ x,     // [M, K]
     const bf16* __restrict__ w,     // [N, K]
@@ -52,11 +54,15 @@ __global__ __launch_bounds__(BLOCK) void skinny_gemm_kernel(
     float* __restrict__ partial,    // [n_split, M, N] when SPLIT
     int M, int N, int K, int k_per) {
   constexpr int R = MT * 16 + 64;            // rows of a buffer: x, then w
-  constexpr int CPW = R / 16;                // copies of four rows per wave
+  constexpr int SL = XK / 8, RPC = 64 / SL;  // slots of a row, rows of a copy
+  constexpr int CPW = R / RPC / 4;           // copies per wave
+  static_assert(CPW * RPC * 4 == R);
+  auto turn = [](int r) { return SL == 16 ? r & 15 : (r >> 1) & 7; };
   __shared__ bf16 lds[NB][R][XK];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, quad = lane >> 4;
-  const int n0 = blockIdx.x * 64 + wave * 16;
+  const int n0 = GLU ? blockIdx.x * 32 + wave * 8
+                     : blockIdx.x * 64 + wave * 16;
   const int kb = SPLIT ? blockIdx.y * k_per : 0;
   const int ke = SPLIT ? min(K, kb + k_per) : K;
 
@@ -64,11 +70,13 @@ __global__ __launch_bounds__(BLOCK) void skinny_gemm_kernel(
   int off[CPW];
 #pragma unroll
   for (int g = 0; g < CPW; ++g) {
-    const int r = (wave * CPW + g) * 4 + quad;
-    src[g] = r < MT * 16
-                 ? x + (int64_t)min(r, M - 1) * K
-                 : w + ((int64_t)blockIdx.x * 64 + r - MT * 16) * K;
-    off[g] = (col ^ (r & 15)) * 8;
+    const int r = (wave * CPW + g) * RPC + lane / SL, wr = r - MT * 16;
+    const int64_t wrow =
+        GLU ? blockIdx.x * 32 + (wr >> 4) * 8 + (wr & 7) +
+                  (wr & 8 ? N / 2 : 0)
+            : blockIdx.x * 64 + wr;
+    src[g] = wr < 0 ? x + (int64_t)min(r, M - 1) * K : w + wrow * K;
+    off[g] = (lane % SL ^ turn(r)) * 8;
   }
   auto copy = [&](int i) {
     const int k0 = kb + i * XK;
@@ -78,14 +86,14 @@ __global__ __launch_bounds__(BLOCK) void skinny_gemm_kernel(
           (const __attribute__((address_space(1))) void*)(
               src[g] + min(k0 + off[g], K - 8)),
           (__attribute__((address_space(3))) void*)(
-              &lds[i & (NB - 1)][(wave * CPW + g) * 4][0]),
+              &lds[i & (NB - 1)][(wave * CPW + g) * RPC][0]),
           16, 0, 0);
   };
   f32x4 acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
   auto product = [&](int buf, int t) {       // 32 k
-    const int s = ((t * 4 + quad) ^ col) * 8;
+    const int s = ((t * 4 + quad) ^ turn(col)) * 8;
     const bf16x8_t wf = *reinterpret_cast<const bf16x8_t*>(
         &lds[buf][MT * 16 + wave * 16 + col][s]);
 #pragma unroll
@@ -120,6 +128,23 @@ __global__ __launch_bounds__(BLOCK) void skinny_gemm_kernel(
       product(whole & (NB - 1), t);
   }
 
+  if (GLU) {                                 // quads 0, 1 gate, 2, 3 up
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      bf16x4_t o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float g = bf2f(f2bf(acc[m][r]));
+        const float u = __shfl_xor(g, 32, 64);
+        o[r] = (__bf16)(g / (1.f + __expf(-g)) * u);
+      }
+      const int row = m * 16 + col;
+      if (quad < 2 && row < M)
+        *reinterpret_cast<bf16x4_t*>(out + (int64_t)row * (N / 2) + n0 +
+                                     quad * 4) = o;
+    }
+    return;
+  }
   // lane: columns n0 + quad * 4 + 0..3 of row m * 16 + col
   const int n = n0 + quad * 4;
   f32x4 b = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -176,28 +201,57 @@ void tl_gemm_reduce(const void* partial, const void* bias, void* out,
 
 // partial: scratch [n_split * M * N] floats (only used when n_split > 1; out
 // null then: the cuts are left for the caller to sum)
+//
+// Uncut products of more than 16 rows have blocks enough for two per CU, which
+// steps of 64 k leave the LDS for (151936 x 4096, 32 / 48 / 64 rows: 252 / 270
+// / 284 us with steps of 128, 246 / 260 / 272 with 64); with cuts, or for 16
+// rows, longer steps are as good or better (6144 x 4096, 32 rows: 14.7, 15.3).
 void tl_skinny_gemm(const void* x, const void* w, const void* bias,
                     void* out, void* partial, int M, int N, int K,
                     int n_split, int k_per, hipStream_t stream) {
   const dim3 grid(N / 64, n_split), block(BLOCK);
-#define TL_SG(MT)                                                            \
+#define TL_SG(MT, XK)                                                            \
   do {                                                                       \
     if (n_split > 1)                                                         \
-      hipLaunchKernelGGL((skinny_gemm_kernel<MT, 1>), grid, block, 0,        \
+      hipLaunchKernelGGL((skinny_gemm_kernel<MT, XK, 1, 0>), grid, block, 0,        \
                          stream, (const bf16*)x, (const bf16*)w, nullptr,    \
                          nullptr, (float*)partial, M, N, K, k_per);          \
     else                                                                     \
-      hipLaunchKernelGGL((skinny_gemm_kernel<MT, 0>), grid, block, 0,        \
+      hipLaunchKernelGGL((skinny_gemm_kernel<MT, XK, 0, 0>), grid, block, 0,        \
                          stream, (const bf16*)x, (const bf16*)w,             \
                          (const bf16*)bias, (bf16*)out, nullptr, M, N, K,    \
                          K);                                                 \
   } while (0)
-  if (M <= 16) TL_SG(1);
-  else if (M <= 32) TL_SG(2);
-  else TL_SG(4);
+  if (M <= 16) {
+    TL_SG(1, 128);
+  } else if (n_split == 1) {
+    if (M <= 32) TL_SG(2, 64);
+    else TL_SG(4, 64);
+  } else {
+    if (M <= 32) TL_SG(2, 128);
+    else if (M <= 48) TL_SG(3, 128);
+    else TL_SG(4, 128);
+  }
 #undef TL_SG
   if (n_split > 1 && out)
     tl_gemm_reduce(partial, bias, out, (int64_t)M * N, N, n_split, stream);
+}
+
+// out [M, N / 2] = silu(x gate^T) (x up^T), w = [gate; up] [N, K]; M <= 64,
+// N a multiple of 64. Against the product and the activation as two launches
+// (the library's, 37888 x 3584 / 28672 x 4096): 1 row 55 / 61 -> 50 / 45 us, 32
+// rows 57 / 54 -> 55 / 46, 64 rows 64 / 55 -> 66 / 52: above 32 rows the caller
+// has N / 64 blocks fit one round of two per CU.
+void tl_skinny_glu(const void* x, const void* w, void* out, int M, int N,
+                   int K, hipStream_t stream) {
+#define TL_SG(MT, XK)                                                        \
+  hipLaunchKernelGGL((skinny_gemm_kernel<MT, XK, 0, 1>), dim3(N / 64),       \
+                     dim3(BLOCK), 0, stream, (const bf16*)x, (const bf16*)w, \
+                     nullptr, (bf16*)out, nullptr, M, N, K, K)
+  if (M <= 16) TL_SG(1, 128);
+  else if (M <= 32) TL_SG(2, 64);
+  else TL_SG(4, 64);
+#undef TL_SG
 }
 
 }  // extern "C"

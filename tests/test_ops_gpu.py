@@ -1046,3 +1046,25 @@ def test_tl_gemm_large_tiles(N, K):
                      for t in x.split(48)])
     for M in (128, 129, 256, 257, 384, 385, 512, 513):
         assert torch.equal(C.skinny_gemm(x[:M].contiguous(), w, b), few[:M])
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("N,K", [(64, 32), (192, 544), (16384, 160)])
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 48, 49, 64])
+def test_skinny_glu(N, K, M):
+    """The activation inside the product: the bits of the two in turn (one
+    cut at these K: up to 32 k steps of one order), and fp64 (gate, up and
+    result rounded to bf16, 2^-9 each: 2-norm error under 8e-3)."""
+    ops = _ext()
+    C = ops._require_ext()
+    torch.manual_seed(N + M)
+    w = torch.randn(N, K, device=DEV, dtype=torch.bfloat16) / K ** 0.5
+    x = torch.randn(M, K, device=DEV, dtype=torch.bfloat16)
+    out = C.skinny_glu(x, w)
+    g, u = (x.double() @ w.double().t()).chunk(2, -1)
+    want = torch.nn.functional.silu(g) * u
+    assert (out.double() - want).norm() / want.norm() < 8e-3
+    if N >= 16384:
+        assert torch.equal(out, C.swiglu_fused(C.skinny_gemm(x, w, None)))
+        assert ops.serving_glu(x, w)
+        assert torch.equal(ops.linear_swiglu(x, w), out)
