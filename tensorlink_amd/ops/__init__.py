@@ -636,7 +636,37 @@ def sample_token(logits, *, temperature=1.0, top_p=1.0, top_k=0,
 
 
 moe_topk_router = ref.moe_topk_router
-causal_lm_loss = ref.causal_lm_loss
+class _CausalCEFn(torch.autograd.Function):
+    """Shifted cross entropy straight on bf16 logits (sums in fp32): one
+    pass over them each way, no shifted or fp32 copy."""
+
+    @staticmethod
+    def forward(ctx, logits, labels, ignore_index):
+        logits, labels = logits.contiguous(), labels.contiguous()
+        loss, lse, mean = _require_ext().ce_fwd(logits, labels, ignore_index)
+        ctx.save_for_backward(logits, labels, lse, mean)
+        ctx.ignore_index = ignore_index
+        return loss.clone()
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dloss):
+        logits, labels, lse, mean = ctx.saved_tensors
+        return _require_ext().ce_bwd(
+            logits, labels, lse, mean, dloss.float().contiguous(),
+            ctx.ignore_index), None, None
+
+
+def causal_lm_loss(logits: torch.Tensor, labels: torch.Tensor,
+                   ignore_index: int = -100) -> torch.Tensor:
+    """Shifted CE loss like HF CausalLM (logits [B,S,V], labels [B,S])."""
+    if (logits.is_cuda and logits.dtype == torch.bfloat16
+            and logits.dim() == 3 and logits.numel() > 0
+            and logits.shape[1] > 1 and labels.is_cuda
+            and labels.dtype == torch.int64
+            and labels.shape == logits.shape[:2]):
+        return _CausalCEFn.apply(logits, labels, ignore_index)
+    return ref.causal_lm_loss(logits, labels, ignore_index)
 rope_cos_sin = ref.rope_cos_sin
 
 

@@ -43,6 +43,12 @@ void tl_rope_rows(void* qkv, void* q, void* k, void* v, const void* positions,
                   int bwd, hipStream_t stream);
 void tl_skinny_glu(const void* x, const void* w, void* out, int M, int N,
                    int K, hipStream_t stream);
+void tl_ce_fwd(const void* logits, const void* labels, void* lse, void* loss,
+               void* mean, int64_t rows, int S, int V, int64_t ignore,
+               hipStream_t stream);
+void tl_ce_bwd(const void* logits, const void* labels, const void* lse,
+               const void* mean, const void* dloss, void* dx, int64_t rows,
+               int S, int V, int64_t ignore, hipStream_t stream);
 void tl_add_norm(const void* x, const void* partial, int n_split,
                  const void* residual, const void* w, void* r_out, void* y,
                  int64_t M, int H, int rounded, float eps,
@@ -473,6 +479,49 @@ Tensor rope_merge(Tensor dq, Tensor dk, Tensor dv, Tensor positions,
   return out;
 }
 
+static void check_ce(const Tensor& logits, const Tensor& labels) {
+  CHECK_IN(logits, torch::kBFloat16);
+  CHECK_IN(labels, torch::kLong);
+  TORCH_CHECK(logits.dim() == 3 && labels.dim() == 2 &&
+                  labels.size(0) == logits.size(0) &&
+                  labels.size(1) == logits.size(1) && logits.numel() > 0 &&
+                  logits.size(2) < (1 << 30) && labels.size(1) < (1 << 30) &&
+                  labels.numel() < (1ll << 31),
+              "logits [B, S, V] and labels [B, S] mismatch");
+}
+
+// (mean loss over the labelled rows, log-sum-exp [B, S], [mean, count])
+std::vector<Tensor> ce_fwd(Tensor logits, Tensor labels, int64_t ignore) {
+  check_ce(logits, labels);
+  auto f32 = logits.options().dtype(torch::kFloat);
+  auto lse = torch::empty(labels.sizes(), f32);
+  auto loss = torch::empty(labels.sizes(), f32);
+  auto mean = torch::empty({2}, f32);
+  tl_ce_fwd(logits.data_ptr(), labels.data_ptr(), lse.data_ptr(),
+            loss.data_ptr(), mean.data_ptr(), labels.numel(),
+            (int)labels.size(1), (int)logits.size(2), ignore, cur_stream());
+  return {mean.select(0, 0), lse, mean};
+}
+
+Tensor ce_bwd(Tensor logits, Tensor labels, Tensor lse, Tensor mean,
+              Tensor dloss, int64_t ignore) {
+  check_ce(logits, labels);
+  CHECK_IN(lse, torch::kFloat);
+  CHECK_IN(mean, torch::kFloat);
+  CHECK_IN(dloss, torch::kFloat);
+  TORCH_CHECK(lse.numel() == labels.numel() && mean.numel() == 2 &&
+                  dloss.numel() == 1,
+              "saved shapes mismatch");
+  // rows of any length: the gradient starts at the logits' offset from 16
+  const int64_t off = (int64_t)(((uintptr_t)logits.data_ptr() & 15) / 2);
+  auto buf = torch::empty({off + logits.numel()}, logits.options());
+  auto dx = buf.narrow(0, off, logits.numel()).view(logits.sizes());
+  tl_ce_bwd(logits.data_ptr(), labels.data_ptr(), lse.data_ptr(),
+            mean.data_ptr(), dloss.data_ptr(), dx.data_ptr(), labels.numel(),
+            (int)labels.size(1), (int)logits.size(2), ignore, cur_stream());
+  return dx;
+}
+
 // Split-K policy SHARED by the streaming (M<=64) and tiled (M>64) GEMM
 // kernels. It depends only on (N, K) — never M — so a row's accumulation
 // (split boundaries + s-ordered reduce) is bitwise identical at every M:
@@ -786,6 +835,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
   mod.def("adamw_", &adamw_, "fused AdamW step");
   mod.def("swiglu_fused_bwd", &swiglu_fused_bwd,
           "gradient of swiglu_fused as one tensor");
+  mod.def("ce_fwd", &ce_fwd, "shifted causal-LM cross entropy");
+  mod.def("ce_bwd", &ce_bwd, "its gradient in the logits' layout");
   mod.def("rope_split", &rope_split,
           "fused projection rows to rotated q, k, and v");
   mod.def("rope_merge", &rope_merge,

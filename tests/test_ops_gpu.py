@@ -1068,3 +1068,56 @@ def test_skinny_glu(N, K, M):
         assert torch.equal(out, C.swiglu_fused(C.skinny_gemm(x, w, None)))
         assert ops.serving_glu(x, w)
         assert torch.equal(ops.linear_swiglu(x, w), out)
+
+
+@pytest.mark.parametrize("B,S,V", [
+    (1, 2, 1), (3, 5, 7), (2, 9, 517), (1, 4, 4096), (2, 33, 50257)])
+@pytest.mark.parametrize("offset", [0, 1, 8])
+def test_causal_lm_loss_kernel(B, S, V, offset):
+    """Rows of any length and alignment against fp64: the loss is summed in
+    fp32; its gradient is rounded to bf16, at most 2^-8 = 3.9e-3 of each
+    element and so of the 2-norm (few elements, one per row, make up most of
+    it, so nothing averages out). Some labels are ignored, some logits
+    -inf."""
+    ops = _ext()
+    torch.manual_seed(V + S)
+    buf = torch.randn(offset + B * S * V, device=DEV,
+                      dtype=torch.bfloat16) * 3
+    x = buf[offset:].view(B, S, V)
+    if V > 64:
+        x[:, :, 5:40] = -math.inf
+    labels = torch.randint(V, (B, S), device=DEV)
+    labels[(labels >= 5) & (labels < 40)] = 0 if V > 64 else 1 % V
+    if S > 4:
+        labels[0, 2] = -100
+    x.requires_grad_(True)
+    loss = ops.causal_lm_loss(x, labels)
+    loss.backward(torch.tensor(0.5, device=DEV))
+    xd = x.detach().double().requires_grad_(True)
+    want = torch.nn.functional.cross_entropy(
+        xd[:, :-1].reshape(-1, V), labels[:, 1:].reshape(-1))
+    want.backward(torch.tensor(0.5, device=DEV, dtype=torch.double))
+    assert loss.dtype == torch.float32 and loss.dim() == 0
+    assert abs(float(loss) - float(want)) <= 2e-6 * max(1., float(want))
+    err = (x.grad.double() - xd.grad).norm()
+    assert err <= 4e-3 * xd.grad.norm()
+    assert (x.grad[:, -1] == 0).all()
+
+
+def test_causal_lm_loss_kernel_without_labels():
+    """No label left is 0 / 0 and no gradient; NaN and labels outside of the
+    vocabulary are not passed over."""
+    ops = _ext()
+    x = torch.randn(1, 4, 33, device=DEV, dtype=torch.bfloat16)
+    y = torch.full((1, 4), -100, device=DEV)
+    x.requires_grad_(True)
+    loss = ops.causal_lm_loss(x, y)
+    loss.backward()
+    assert torch.isnan(loss) and (x.grad == 0).all()
+    for bad in (-1, 33):
+        y[0, 2] = bad
+        assert torch.isnan(ops.causal_lm_loss(x, y))
+    y[0, 2] = 3
+    with torch.no_grad():
+        x[0, 1, 7] = math.nan
+    assert torch.isnan(ops.causal_lm_loss(x, y))
