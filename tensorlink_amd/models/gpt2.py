@@ -22,7 +22,7 @@ import torch.nn.functional as F
 
 from tensorlink_amd import ops
 from tensorlink_amd.models.configs import ModelConfig
-from tensorlink_amd.models.dense import KVCache
+from tensorlink_amd.models.dense import KVCache, _unwatched
 
 
 def gpt2_config(name: str = "gpt2-small") -> ModelConfig:
@@ -40,6 +40,22 @@ def gpt2_config(name: str = "gpt2-small") -> ModelConfig:
         architecture="gpt2", rms_norm_eps=1e-5)
 
 
+def _rows(training: bool, x: torch.Tensor, *modules: nn.Module) -> bool:
+    """A training step on the GPU through plain, unwatched layers with
+    biases: their kernels are called directly (ops, train_rows.hip)."""
+    return training and ops.train_rows_fit(x) and all(
+        type(m) in (nn.Linear, nn.LayerNorm) and _unwatched(m)
+        and m.bias is not None and ops.train_rows_fit(m.weight, m.bias)
+        and (type(m) is nn.Linear or m.weight.shape[-1] <= 2048)
+        for m in modules)
+
+
+def _linear(m: nn.Linear, x: torch.Tensor, training: bool) -> torch.Tensor:
+    if _rows(training, x, m):
+        return ops.linear_bias(x, m.weight, m.bias)
+    return m(x)
+
+
 class Gpt2Attention(nn.Module):
     def __init__(self, config: ModelConfig):
         super().__init__()
@@ -53,8 +69,12 @@ class Gpt2Attention(nn.Module):
     def forward(self, x, kv_cache: Optional[KVCache], layer_idx: int,
                 positions, training: bool):
         B, S, H = x.shape
-        qkv = self.c_attn(x)
-        q, k, v = qkv.split(H, dim=-1)
+        qkv = _linear(self.c_attn, x, training)
+        if training:
+            q, k, v = ops.split_rows(qkv.view(B * S, -1), self.n_heads,
+                                     self.n_heads)
+        else:
+            q, k, v = qkv.split(H, dim=-1)
         q = q.view(B, S, self.n_heads, self.head_dim)
         k = k.view(B, S, self.n_heads, self.head_dim)
         v = v.view(B, S, self.n_heads, self.head_dim)
@@ -78,7 +98,7 @@ class Gpt2Attention(nn.Module):
                 out = ops.attention_prefill_cache(
                     q, kv_cache.k[layer_idx], kv_cache.v[layer_idx], off + S,
                     scale=self.scale, block_table=table)
-        return self.c_proj(out.reshape(B, S, H))
+        return _linear(self.c_proj, out.reshape(B, S, H), training)
 
 
 class Gpt2Block(nn.Module):
@@ -92,6 +112,13 @@ class Gpt2Block(nn.Module):
         self.c_proj = nn.Linear(config.intermediate_size, h)
 
     def forward(self, x, kv_cache, layer_idx, positions, training):
+        if _rows(training, x, self.ln_1, self.ln_2, self.c_fc, self.c_proj):
+            n1, n2, fc, proj = self.ln_1, self.ln_2, self.c_fc, self.c_proj
+            a = self.attn(ops.layernorm(x, n1.weight, n1.bias, n1.eps),
+                          kv_cache, layer_idx, positions, training)
+            x, h = ops.add_layernorm(x, a, n2.weight, n2.bias, n2.eps)
+            h = ops.linear_bias(h, fc.weight, fc.bias, gelu=True)
+            return x + ops.linear_bias(h, proj.weight, proj.bias)
         x = x + self.attn(self.ln_1(x), kv_cache, layer_idx, positions,
                           training)
         x = x + self.c_proj(F.gelu(self.c_fc(self.ln_2(x)),

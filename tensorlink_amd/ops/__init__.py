@@ -281,6 +281,124 @@ def rope_rows(qkv: torch.Tensor, positions: torch.Tensor,
     return q, k, v
 
 
+class _RowsFn(torch.autograd.Function):
+    """Projection rows to q, k and v, one pass each way."""
+
+    @staticmethod
+    def forward(ctx, qkv, n_heads, n_kv, D):
+        return tuple(_require_ext().rows_split(qkv.contiguous(), n_heads,
+                                               n_kv, D))
+
+    @staticmethod
+    def backward(ctx, dq, dk, dv):
+        return (_require_ext().rows_merge(dq.contiguous(), dk.contiguous(),
+                                          dv.contiguous()), None, None, None)
+
+
+def split_rows(qkv: torch.Tensor, n_heads: int, n_kv: int):
+    """Rows [T, (n_heads + 2 n_kv) * D] to q [T, n_heads, D] and k, v
+    [T, n_kv, D]."""
+    D = qkv.shape[-1] // (n_heads + 2 * n_kv)
+    if qkv.is_cuda and qkv.dtype == torch.bfloat16 and D % 16 == 0:
+        return _RowsFn.apply(qkv, n_heads, n_kv, D)
+    return tuple(t.reshape(t.shape[0], -1, D) for t in qkv.split(
+        [n_heads * D, n_kv * D, n_kv * D], dim=-1))
+
+
+# ---------------------------------------------------------------------------
+# Training rows of layers with biases and layer norms
+# ---------------------------------------------------------------------------
+def train_rows_fit(*tensors: torch.Tensor) -> bool:
+    """The kernels of train_rows.hip: bf16 rows of whole 16-byte pieces, the
+    arguments' own types (no autocast), gradients of first order."""
+    return (torch.is_grad_enabled() and not torch.is_autocast_enabled()
+            and all(t.is_cuda and t.dtype == torch.bfloat16
+                    and t.shape[-1] % 8 == 0 and t.numel() > 0
+                    for t in tensors))
+
+
+class _LinearBiasFn(torch.autograd.Function):
+    """y = x W^T + b, with gelu (tanh form) behind it if asked to; the bias's
+    gradient and gelu's in one pass over the rows."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, gelu):
+        z = torch.nn.functional.linear(x, weight, bias)
+        ctx.gelu = gelu
+        ctx.save_for_backward(x, weight, z if gelu else None)
+        return torch.nn.functional.gelu(z, approximate="tanh") if gelu else z
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dy):
+        x, weight, z = ctx.saved_tensors
+        dy = dy.contiguous()
+        if ctx.gelu:
+            dy, db = _require_ext().bias_grad(dy, z)
+        elif ctx.needs_input_grad[2]:
+            db, = _require_ext().bias_grad(dy, None)
+        else:
+            db = None
+        rows = dy.view(-1, dy.shape[-1])
+        dx = dy @ weight if ctx.needs_input_grad[0] else None
+        dw = (rows.t() @ x.reshape(-1, x.shape[-1])
+              if ctx.needs_input_grad[1] else None)
+        return dx, dw, db if ctx.needs_input_grad[2] else None, None
+
+
+def linear_bias(x, weight, bias, gelu: bool = False):
+    """Training: x W^T + b, gelu of it if asked to. For tensors that
+    train_rows_fit() takes."""
+    return _LinearBiasFn.apply(x, weight, bias, gelu)
+
+
+class _LayerNormFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, weight, bias, eps):
+        x = x.contiguous()
+        y, mean, rstd = _require_ext().layernorm_fwd(
+            x, None, weight.contiguous(), bias.contiguous(), eps)
+        ctx.save_for_backward(x, weight, mean, rstd)
+        return y
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dy):
+        x, weight, mean, rstd = ctx.saved_tensors
+        return (*_require_ext().layernorm_bwd(
+            dy.contiguous(), None, x, weight.contiguous(), mean, rstd), None)
+
+
+class _AddLayerNormFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, a, weight, bias, eps):
+        y, mean, rstd, r = _require_ext().layernorm_fwd(
+            x.contiguous(), a.contiguous(), weight.contiguous(),
+            bias.contiguous(), eps)
+        ctx.save_for_backward(r, weight, mean, rstd)
+        return r, y
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dr, dy):
+        r, weight, mean, rstd = ctx.saved_tensors
+        d, dw, db = _require_ext().layernorm_bwd(
+            dy.contiguous(), dr.contiguous(), r, weight.contiguous(), mean,
+            rstd)
+        return d, d, dw, db, None
+
+
+def layernorm(x, weight, bias, eps: float):
+    """Training LayerNorm of rows up to 2048 wide that train_rows_fit()
+    takes."""
+    return _LayerNormFn.apply(x, weight, bias, eps)
+
+
+def add_layernorm(x, a, weight, bias, eps: float):
+    """(r, LayerNorm(r)) with r = x + a, and one gradient for both."""
+    return _AddLayerNormFn.apply(x, a, weight, bias, eps)
+
+
 # ---------------------------------------------------------------------------
 # SwiGLU
 # ---------------------------------------------------------------------------

@@ -49,6 +49,19 @@ void tl_ce_fwd(const void* logits, const void* labels, void* lse, void* loss,
 void tl_ce_bwd(const void* logits, const void* labels, const void* lse,
                const void* mean, const void* dloss, void* dx, int64_t rows,
                int S, int V, int64_t ignore, hipStream_t stream);
+void tl_reduce_partials(const void* partials, void* out, int P, int64_t H,
+                        hipStream_t stream);
+int tl_bias_grad_rows(int64_t M, int N);
+void tl_bias_grad(const void* dy, const void* z, void* dz, void* partial,
+                  int64_t M, int N, int per, hipStream_t stream);
+void tl_layernorm_fwd(const void* x, const void* a, const void* w,
+                      const void* b, void* r_out, void* y, void* mean,
+                      void* rstd, int64_t M, int W, float eps,
+                      hipStream_t stream);
+void tl_layernorm_bwd(const void* dy, const void* dr, const void* r,
+                      const void* w, const void* mean, const void* rstd,
+                      void* dx, void* partial, int64_t M, int W, int blocks,
+                      hipStream_t stream);
 void tl_add_norm(const void* x, const void* partial, int n_split,
                  const void* residual, const void* w, void* r_out, void* y,
                  int64_t M, int H, int rounded, float eps,
@@ -522,6 +535,125 @@ Tensor ce_bwd(Tensor logits, Tensor labels, Tensor lse, Tensor mean,
   return dx;
 }
 
+// projection rows [T, (Hq + 2 Hkv) D] to q, k and v, and back
+std::vector<Tensor> rows_split(Tensor qkv, int64_t Hq, int64_t Hkv,
+                               int64_t D) {
+  CHECK_IN(qkv, torch::kBFloat16);
+  TORCH_CHECK(qkv.dim() == 2 && qkv.size(1) == (Hq + 2 * Hkv) * D &&
+                  D % 16 == 0,
+              "qkv width mismatch");
+  const int64_t T = qkv.size(0);
+  auto q = torch::empty({T, Hq, D}, qkv.options());
+  auto k = torch::empty({T, Hkv, D}, qkv.options());
+  auto v = torch::empty_like(k);
+  tl_rope_rows(qkv.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+               nullptr, nullptr, T, (int)Hq, (int)Hkv, (int)D, 0,
+               cur_stream());
+  return {q, k, v};
+}
+
+Tensor rows_merge(Tensor dq, Tensor dk, Tensor dv) {
+  CHECK_IN(dq, torch::kBFloat16);
+  CHECK_IN(dk, torch::kBFloat16);
+  CHECK_IN(dv, torch::kBFloat16);
+  TORCH_CHECK(dq.dim() == 3 && dk.dim() == 3 && dk.size(0) == dq.size(0) &&
+                  dk.size(2) == dq.size(2) && dv.sizes() == dk.sizes() &&
+                  dq.size(2) % 16 == 0,
+              "gradient shapes mismatch");
+  const int64_t T = dq.size(0), Hq = dq.size(1), Hkv = dk.size(1);
+  const int64_t D = dq.size(2);
+  auto out = torch::empty({T, (Hq + 2 * Hkv) * D}, dq.options());
+  tl_rope_rows(out.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+               nullptr, nullptr, T, (int)Hq, (int)Hkv, (int)D, 1,
+               cur_stream());
+  return out;
+}
+
+// {column sums of dy}, or with z {dz = dy gelu'(z), column sums of dz}
+std::vector<Tensor> bias_grad(Tensor dy, c10::optional<Tensor> z) {
+  CHECK_IN(dy, torch::kBFloat16);
+  const int64_t N = dy.size(-1), M = N ? dy.numel() / N : 0;
+  TORCH_CHECK(M > 0 && N % 8 == 0, "rows must be a multiple of 8 wide");
+  const int per = tl_bias_grad_rows(M, (int)N);
+  const int P = (int)((M + per - 1) / per);
+  auto partial = torch::empty({P, N}, dy.options().dtype(torch::kFloat));
+  auto db = torch::empty({N}, dy.options());
+  Tensor dz;
+  if (z.has_value()) {
+    CHECK_IN(z.value(), torch::kBFloat16);
+    TORCH_CHECK(z->sizes() == dy.sizes(), "shapes differ");
+    dz = torch::empty_like(dy);
+  }
+  tl_bias_grad(dy.data_ptr(), z.has_value() ? z->data_ptr() : nullptr,
+               z.has_value() ? dz.data_ptr() : nullptr, partial.data_ptr(),
+               M, (int)N, per, cur_stream());
+  tl_reduce_partials(partial.data_ptr(), db.data_ptr(), P, N, cur_stream());
+  if (z.has_value()) return {dz, db};
+  return {db};
+}
+
+static int64_t check_ln(const Tensor& x, const Tensor& w) {
+  CHECK_IN(x, torch::kBFloat16);
+  CHECK_IN(w, torch::kBFloat16);
+  const int64_t W = x.size(-1);
+  TORCH_CHECK(W % 8 == 0 && W <= 2048 && w.numel() == W && x.numel() > 0,
+              "rows must be a multiple of 8 wide, at most 2048");
+  return W;
+}
+
+// (y, mean, rstd) or with a (y, mean, rstd, r = x + a)
+std::vector<Tensor> layernorm_fwd(Tensor x, c10::optional<Tensor> a, Tensor w,
+                                  Tensor b, double eps) {
+  const int64_t W = check_ln(x, w), M = x.numel() / W;
+  CHECK_IN(b, torch::kBFloat16);
+  TORCH_CHECK(b.numel() == W, "norm bias size mismatch");
+  auto f32 = x.options().dtype(torch::kFloat);
+  auto y = torch::empty_like(x);
+  auto mean = torch::empty({M}, f32), rstd = torch::empty({M}, f32);
+  Tensor r;
+  if (a.has_value()) {
+    CHECK_IN(a.value(), torch::kBFloat16);
+    TORCH_CHECK(a->sizes() == x.sizes(), "shapes differ");
+    r = torch::empty_like(x);
+  }
+  tl_layernorm_fwd(x.data_ptr(), a.has_value() ? a->data_ptr() : nullptr,
+                   w.data_ptr(), b.data_ptr(),
+                   a.has_value() ? r.data_ptr() : nullptr, y.data_ptr(),
+                   mean.data_ptr(), rstd.data_ptr(), M, (int)W, (float)eps,
+                   cur_stream());
+  if (a.has_value()) return {y, mean, rstd, r};
+  return {y, mean, rstd};
+}
+
+// (gradient of r, dw, db); dr: what comes along r itself
+std::vector<Tensor> layernorm_bwd(Tensor dy, c10::optional<Tensor> dr,
+                                  Tensor r, Tensor w, Tensor mean,
+                                  Tensor rstd) {
+  const int64_t W = check_ln(r, w), M = r.numel() / W;
+  CHECK_IN(dy, torch::kBFloat16);
+  CHECK_IN(mean, torch::kFloat);
+  CHECK_IN(rstd, torch::kFloat);
+  TORCH_CHECK(dy.sizes() == r.sizes() && mean.numel() == M &&
+                  rstd.numel() == M,
+              "saved shapes mismatch");
+  if (dr.has_value()) {
+    CHECK_IN(dr.value(), torch::kBFloat16);
+    TORCH_CHECK(dr->sizes() == r.sizes(), "shapes differ");
+  }
+  const int blocks = (int)std::min<int64_t>(256, (M + 3) / 4);
+  auto dx = torch::empty_like(r);
+  auto partial = torch::empty({blocks, 2 * W},
+                              r.options().dtype(torch::kFloat));
+  auto dwb = torch::empty({2, W}, r.options());
+  tl_layernorm_bwd(dy.data_ptr(), dr.has_value() ? dr->data_ptr() : nullptr,
+                   r.data_ptr(), w.data_ptr(), mean.data_ptr(),
+                   rstd.data_ptr(), dx.data_ptr(), partial.data_ptr(), M,
+                   (int)W, blocks, cur_stream());
+  tl_reduce_partials(partial.data_ptr(), dwb.data_ptr(), blocks, 2 * W,
+                     cur_stream());
+  return {dx, dwb.select(0, 0), dwb.select(0, 1)};
+}
+
 // Split-K policy SHARED by the streaming (M<=64) and tiled (M>64) GEMM
 // kernels. It depends only on (N, K) — never M — so a row's accumulation
 // (split boundaries + s-ordered reduce) is bitwise identical at every M:
@@ -837,6 +969,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
           "gradient of swiglu_fused as one tensor");
   mod.def("ce_fwd", &ce_fwd, "shifted causal-LM cross entropy");
   mod.def("ce_bwd", &ce_bwd, "its gradient in the logits' layout");
+  mod.def("rows_split", &rows_split, "projection rows to q, k, and v");
+  mod.def("rows_merge", &rows_merge, "its backward");
+  mod.def("bias_grad", &bias_grad, "column sums (and GELU's gradient)");
+  mod.def("layernorm_fwd", &layernorm_fwd, "(add and) LayerNorm");
+  mod.def("layernorm_bwd", &layernorm_bwd, "its backward");
   mod.def("rope_split", &rope_split,
           "fused projection rows to rotated q, k, and v");
   mod.def("rope_merge", &rope_merge,

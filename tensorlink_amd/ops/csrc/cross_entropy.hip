@@ -9,8 +9,7 @@
 //
 // 4 x 512 x 50257: shifted copy, conversion to fp32, log-softmax, selection
 // and all of it backwards were 1050 us in 12 launches, and are 200 us in three
-// (49 us forward, 4.2 TB/s; 146 us backward, 2.8 TB/s: the rows' odd starts
-// leave its 16-byte stores unaligned to the 64-byte sectors).
+// (49 us forward, 4.2 TB/s; 146 us backward, 2.8 TB/s).
 
 #include <cstdint>
 

@@ -268,6 +268,14 @@ void launch_fwd(const bf16* x, const bf16* res, const bf16* w, bf16* y,
 
 extern "C" {
 
+// out[h] = the sum of P fp32 slabs, in bf16
+void tl_reduce_partials(const void* partials, void* out, int P, int64_t H,
+                        hipStream_t stream) {
+  hipLaunchKernelGGL(reduce_partials_kernel, dim3((uint32_t)((H + 31) / 32)),
+                     dim3(1024), 0, stream, (const float*)partials,
+                     (bf16*)out, P, H);
+}
+
 void tl_rmsnorm_fwd(const void* x, const void* residual, const void* w,
                     void* y, void* r_out, void* rstd, int64_t N, int H,
                     float eps, hipStream_t stream) {

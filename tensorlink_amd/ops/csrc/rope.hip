@@ -54,7 +54,7 @@ __global__ __launch_bounds__(BLOCK) void rope_rows_kernel(
     bf16* __restrict__ v, const int* __restrict__ positions,
     const float* __restrict__ inv_freq, int Hq, int Hkv, int D) {
   const int64_t token = blockIdx.x;
-  const float pos = (float)positions[token];
+  const float pos = inv_freq ? (float)positions[token] : 0.f;
   const int D2 = D / 2, C = D2 / 8, H = Hq + 2 * Hkv;
   bf16* row = qkv + token * H * D;
   for (int i = threadIdx.x; i < H * C; i += BLOCK) {
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(BLOCK) void rope_rows_kernel(
     bf16* dst = BWD ? row + h * D : part;
     bf16x8 a = *reinterpret_cast<const bf16x8*>(src + d);
     bf16x8 b = *reinterpret_cast<const bf16x8*>(src + d + D2);
-    if (h < Hq + Hkv) {
+    if (inv_freq && h < Hq + Hkv) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         float c, s;
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(BLOCK) void rope_rows_kernel(
 
 extern "C" {
 
-// D a multiple of 16
+// D a multiple of 16; inv_freq null: no rotation
 void tl_rope_rows(void* qkv, void* q, void* k, void* v, const void* positions,
                   const void* inv_freq, int64_t T, int Hq, int Hkv, int D,
                   int bwd, hipStream_t stream) {

@@ -1121,3 +1121,86 @@ def test_causal_lm_loss_kernel_without_labels():
     with torch.no_grad():
         x[0, 1, 7] = math.nan
     assert torch.isnan(ops.causal_lm_loss(x, y))
+
+
+@pytest.mark.parametrize("M,N", [(1, 8), (17, 136), (33, 768), (2100, 1000)])
+def test_linear_bias_gradients(M, N):
+    """Sums in fp32 of rows rounded to bf16 (2^-8 at most), one rounding of
+    the result: against fp64 of the same rounded rows where there is no
+    activation, else 2-norm errors under 1e-2."""
+    ops = _ext()
+    torch.manual_seed(N)
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    dy, z = mk(M, N), mk(M, N) * 2
+    db, = ops._require_ext().bias_grad(dy, None)
+    want = dy.double().sum(0)
+    scale = dy.double().abs().sum(0)
+    assert ((db.double() - want).abs()
+            <= want.abs() * 2 ** -8 + scale * 1e-6).all()
+    dz, db = ops._require_ext().bias_grad(dy, z)
+    zd = z.double().requires_grad_(True)
+    torch.nn.functional.gelu(zd, approximate="tanh").backward(dy.double())
+    assert (dz.double() - zd.grad).norm() < 4e-3 * zd.grad.norm()
+    want, scale = dz.double().sum(0), dz.double().abs().sum(0)
+    assert ((db.double() - want).abs()
+            <= want.abs() * 2 ** -8 + scale * 1e-6).all()
+    K = 64
+    x, w, b = (t.requires_grad_(True) for t in (mk(M, K), mk(N, K), mk(N)))
+    for gelu in (False, True):
+        y = ops.linear_bias(x, w, b, gelu)
+        got = torch.autograd.grad(y, (x, w, b), dy)
+        xd, wd, bd = (t.detach().double().requires_grad_(True)
+                      for t in (x, w, b))
+        yd = torch.nn.functional.linear(xd, wd, bd)
+        if gelu:
+            yd = torch.nn.functional.gelu(yd, approximate="tanh")
+        assert (y.double() - yd).norm() < 1e-2 * yd.norm()
+        for g, d in zip(got, torch.autograd.grad(yd, (xd, wd, bd),
+                                                 dy.double())):
+            assert (g.double() - d).norm() < 1e-2 * d.norm()
+
+
+@pytest.mark.parametrize("M,W", [
+    (1, 8), (3, 512), (5, 520), (1030, 768), (9, 1536), (7, 2048)])
+def test_layernorm_rows(M, W):
+    """Forward and gradients against fp64: results are rounded to bf16 (2^-8
+    at most), sums are fp32. The sum with the residual is the bf16 one."""
+    ops = _ext()
+    torch.manual_seed(W)
+    mk = lambda *s: torch.randn(*s, device=DEV, dtype=torch.bfloat16)
+    x, a, w, b = (t.requires_grad_(True)
+                  for t in (mk(M, W), mk(M, W), mk(W), mk(W)))
+    dy, dr = mk(M, W), mk(M, W)
+    norm = lambda t, w, b: torch.nn.functional.layer_norm(t, (W,), w, b, 1e-5)
+    y = ops.layernorm(x, w, b, 1e-5)
+    got = torch.autograd.grad(y, (x, w, b), dy)
+    xd, wd, bd = (t.detach().double().requires_grad_(True)
+                  for t in (x, w, b))
+    yd = norm(xd, wd, bd)
+    assert (y.double() - yd).norm() < 4e-3 * yd.norm()
+    for g, d in zip(got, torch.autograd.grad(yd, (xd, wd, bd), dy.double())):
+        assert (g.double() - d).norm() < 4e-3 * d.norm()
+    r, y = ops.add_layernorm(x, a, w, b, 1e-5)
+    assert torch.equal(r, x + a)
+    got = torch.autograd.grad((r, y), (x, a, w, b), (dr, dy))
+    assert torch.equal(got[0], got[1])
+    rd = r.detach().double().requires_grad_(True)
+    yd = norm(rd, wd, bd)
+    assert (y.double() - yd).norm() < 4e-3 * yd.norm()
+    want = torch.autograd.grad((rd, yd), (rd, wd, bd),
+                               (dr.double(), dy.double()))
+    for g, d in zip((got[0], *got[2:]), want):
+        assert (g.double() - d).norm() < 4e-3 * d.norm()
+
+
+def test_split_rows():
+    ops = _ext()
+    T, Hq, Hkv, D = 5, 3, 2, 48
+    rows = torch.randn(T, (Hq + 2 * Hkv) * D, device=DEV,
+                       dtype=torch.bfloat16, requires_grad=True)
+    parts = ops.split_rows(rows, Hq, Hkv)
+    want = rows.split([Hq * D, Hkv * D, Hkv * D], -1)
+    for p, t in zip(parts, want):
+        assert torch.equal(p.reshape(T, -1), t)
+    torch.autograd.backward(parts, [2 * p.detach() for p in parts])
+    assert torch.equal(rows.grad, 2 * rows)
