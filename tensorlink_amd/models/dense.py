@@ -285,6 +285,8 @@ class MoEMLP(nn.Module):
         kernel (ops/csrc/moe_gemm.hip) can serve this block; None falls
         back to the per-expert loop (CPU, training, fp4)."""
         from tensorlink_amd.models.quant import Fp8Linear
+        if self.top_k > 64 or self.num_experts > 2048:
+            return None                  # the router kernel's limits
         e0 = self.experts[0]
         if isinstance(e0.gate_up_proj, Fp8Linear):
             return "fp8"
