@@ -41,6 +41,13 @@ def _on_gpu(*tensors: torch.Tensor) -> bool:
     return any(t.is_cuda for t in tensors if isinstance(t, torch.Tensor))
 
 
+def _plain_autograd() -> bool:
+    """No function transform (vmap, grad, jvp) or forward-mode level is
+    active: those want torch's own operations."""
+    return (not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0)
+
+
 # ---------------------------------------------------------------------------
 # RMSNorm (autograd-aware)
 # ---------------------------------------------------------------------------
@@ -312,6 +319,7 @@ def train_rows_fit(*tensors: torch.Tensor) -> bool:
     """The kernels of train_rows.hip: bf16 rows of whole 16-byte pieces, the
     arguments' own types (no autocast), gradients of first order."""
     return (torch.is_grad_enabled() and not torch.is_autocast_enabled()
+            and _plain_autograd()
             and all(t.is_cuda and t.dtype == torch.bfloat16
                     and t.shape[-1] % 8 == 0 and t.numel() > 0
                     for t in tensors))
@@ -767,9 +775,12 @@ class _CausalCEFn(torch.autograd.Function):
         return loss.clone()
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, dloss):
         logits, labels, lse, mean = ctx.saved_tensors
+        if torch.is_grad_enabled():      # create_graph: in torch's operations
+            return (*torch.autograd.grad(
+                ref.causal_lm_loss(logits, labels, ctx.ignore_index), logits,
+                dloss, create_graph=True), None, None)
         return _require_ext().ce_bwd(
             logits, labels, lse, mean, dloss.float().contiguous(),
             ctx.ignore_index), None, None
@@ -778,7 +789,8 @@ class _CausalCEFn(torch.autograd.Function):
 def causal_lm_loss(logits: torch.Tensor, labels: torch.Tensor,
                    ignore_index: int = -100) -> torch.Tensor:
     """Shifted CE loss like HF CausalLM (logits [B,S,V], labels [B,S])."""
-    if (logits.is_cuda and logits.dtype == torch.bfloat16
+    if (_plain_autograd()
+            and logits.is_cuda and logits.dtype == torch.bfloat16
             and logits.dim() == 3 and logits.numel() > 0
             and logits.shape[1] > 1 and labels.is_cuda
             and labels.dtype == torch.int64

@@ -1204,3 +1204,25 @@ def test_split_rows():
         assert torch.equal(p.reshape(T, -1), t)
     torch.autograd.backward(parts, [2 * p.detach() for p in parts])
     assert torch.equal(rows.grad, 2 * rows)
+
+
+def test_causal_lm_loss_other_derivatives():
+    """Second derivatives, function transforms and forward mode are torch's,
+    as of the reference."""
+    ops = _ext()
+    from tensorlink_amd.ops import reference as ref
+    torch.manual_seed(3)
+    x = torch.randn(2, 5, 33, device=DEV, dtype=torch.bfloat16)
+    y = torch.randint(33, (2, 5), device=DEV)
+    v = torch.randn_like(x)
+    got = []
+    for loss in (ops.causal_lm_loss, ref.causal_lm_loss):
+        t = x.clone().requires_grad_(True)
+        g, = torch.autograd.grad(loss(t, y), t, create_graph=True)
+        h, = torch.autograd.grad((g * v).sum(), t)
+        with torch.autograd.forward_ad.dual_level():
+            d = torch.autograd.forward_ad.make_dual(x, v)
+            j = torch.autograd.forward_ad.unpack_dual(loss(d, y)).tangent
+        got.append((h, j, torch.func.grad(loss)(x, y)))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
