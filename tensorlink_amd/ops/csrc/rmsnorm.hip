@@ -168,7 +168,8 @@ __global__ __launch_bounds__(1024) void reduce_partials_kernel(
 }
 
 // Narrow rows (a head's 64 to 512 elements): L = H / 8 lanes per row instead
-// of a block, the same sums.
+// of a block, the same sums. 76800 rows of 128: 40 -> 6.8 us forward (5.8
+// TB/s), 250 -> 18 backward.
 template <int L>
 __global__ __launch_bounds__(BLOCK) void rmsnorm_fwd_narrow_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ w,
